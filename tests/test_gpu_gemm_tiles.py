@@ -1,0 +1,64 @@
+"""The GEMM engine's tile kernels at the sizes where they can go wrong: rows
+and columns around every tile edge, K around its chunk and split lengths,
+16-byte loads against operands that are not aligned for them, and a
+bound-exact comparison with numpy.
+
+The products run through the phi2 updates (tt_linalg.f90:315-340): the left
+one multiplies two transposed operands (contiguous along K), the right one a
+row-contiguous operand and a transposed one.  |computed - exact| is at most
+K eps |A| |B| per product to first order; the two chained products and the
+reference's own rounding are covered by 2 (K1 + K2 + 2) eps on the product of
+absolute values.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 1, 1, 1), (15, 17, 16, 1, 33), (64, 64, 64, 2, 64), (65, 63, 127, 1, 129), (128, 96, 40, 3, 97),
+         (130, 31, 1000, 2, 66), (33, 200, 18, 5, 80), (2, 2, 514, 64, 2), (96, 128, 256, 1, 192),
+         (192, 16, 30, 1, 16)]
+
+
+def _run(side, dims, shift):
+    import ttfort
+    lib = ttfort.load()
+    rx1, rx2, ry1, n, ry2 = dims
+    rng = np.random.default_rng(sum(dims))
+    if side == "left":
+        p = rng.standard_normal((ry1, rx1))
+        out_shape = (ry2, rx2)
+    else:
+        p = rng.standard_normal((rx2, ry2))
+        out_shape = (rx1, ry1)
+    x, y = rng.standard_normal((rx1, n, rx2)), rng.standard_normal((ry1, n, ry2))
+
+    def dev(a):   # `shift` doubles into an allocation: 8 bytes off the 16-byte grid when odd
+        d = ttfort.DeviceArray((a.size + shift,))
+        d.upload(np.concatenate([np.zeros(shift), a.reshape(-1, order="F")]))
+        return d
+
+    d = [dev(a) for a in (p, x, y)]
+    out = ttfort.DeviceArray(out_shape)
+    fn = lib.ttf_dphi2_left if side == "left" else lib.ttf_dphi2_right
+    ttfort.check(fn(rx1, rx2, ry1, n, ry2, *[ctypes.c_void_p(a.ptr + 8 * shift) for a in d], out.ptr), lib)
+
+    def chain(p, x, y):
+        if side == "left":
+            return np.einsum("cbj,bja->ca", np.einsum("gb,gjc->cbj", p, y, optimize=True), x, optimize=True)
+        return np.einsum("bjc,gjc->bg", np.einsum("bja,ac->bjc", x, p, optimize=True), y, optimize=True)
+
+    k = (ry1 + rx1 * n) if side == "left" else (rx2 + n * ry2)
+    bound = 2 * (k + 2) * np.finfo(float).eps * chain(abs(p), abs(x), abs(y))
+    return out.numpy(), chain(p, x, y), bound
+
+
+@pytest.mark.parametrize("side", ["left", "right"])
+@pytest.mark.parametrize("dims", SIZES)
+def test_gemm_tile_edges(ttlib, side, dims):
+    aligned, ref, bound = _run(side, dims, 0)
+    assert np.all(np.abs(aligned - ref) <= bound)
+    shifted, _, _ = _run(side, dims, 1)
+    assert np.array_equal(aligned, shifted)   # the same sums in the same order

@@ -2,6 +2,7 @@
 // small-panel kernel for products with a short K and a narrow shared B.
 #include "gemm_mfma.h"
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -95,12 +96,19 @@ static bool panel_eligible(const GemmOp<T>& op) {
 static thread_local bool t_no_tune = false;
 void gemm_no_tuning(bool on) { t_no_tune = on; }
 
+// A tile shape (kTiles below) and the split-K factor ks.
 struct Cfg {
-  int bm, bk, ks;   // tiles bm x bm (or bm x bn), K chunk bk, split-K factor ks
-  int bn = 0;       // 0: square tiles; 80: 64 x 80 tiles, four waves stacked in rows
+  int bm, bn, ks;
 };
 
-static int cfg_bn(const Cfg& c) { return c.bn > 0 ? c.bn : c.bm; }
+// The tile shapes that launch_tiles instantiates.  `rate`: the share of the
+// matrix cores' rate that a chip full of such work-groups reaches with a
+// long K, in hundredths (f64, 16-byte loads), which orders the candidates.
+struct Tile {
+  int bm, bn, threads, rate;
+};
+static const Tile kTiles[] = {{128, 64, 256, 92}, {64, 96, 512, 90}, {64, 80, 256, 84}, {64, 64, 256, 86},
+                              {64, 32, 256, 82},  {32, 32, 256, 70}, {32, 16, 64, 45}};
 
 struct Key {
   int type, M, N, K, nbatch, flags;
@@ -126,8 +134,9 @@ bool g_table_loaded = false;
 }  // namespace
 
 // Persistent tuning table: when TTF_TUNE_FILE names a file, its entries
-// ("type M N K nbatch flags bm bk ks bn" per line; a line without bn means
-// square tiles) are loaded on first use and
+// ("type M N K nbatch flags bm bk ks bn" per line; a line without bn, or
+// with bn 0, means square tiles, and bk is kept for older tables and not
+// used) are loaded on first use and
 // every newly tuned shape is appended, so that separate processes (a timed
 // run and its counter-collection reruns, or successive jobs) launch the same
 // configuration for the same product.  Called with g_tune_mu held.
@@ -149,13 +158,13 @@ static void load_tune_table() {
   while (std::fgets(line, sizeof(line), fp)) {
     Key k{};
     Cfg c{};
+    int bk = 0;
     const int got = std::sscanf(line, "%d %d %d %d %d %d %d %d %d %d", &k.type, &k.M, &k.N, &k.K, &k.nbatch,
-                                &k.flags, &c.bm, &c.bk, &c.ks, &c.bn);
-    if (got == 9) c.bn = 0;
-    const bool valid = (got == 9 || got == 10) && (c.bm == 32 || c.bm == 64) &&
-                       (c.bk == 16 || c.bk == 32 || c.bk == 64) && c.ks >= 1 && c.ks <= 16 &&
-                       (c.bn == 0 || (c.bn == 80 && c.bm == 64 && c.bk <= 32) || (c.bn == 16 && c.bm == 32));
-    if (valid) {
+                                &k.flags, &c.bm, &bk, &c.ks, &c.bn);
+    if (got == 9 || (got == 10 && c.bn == 0)) c.bn = c.bm;
+    bool valid = false;
+    for (const Tile& t : kTiles) valid = valid || (t.bm == c.bm && t.bn == c.bn);
+    if ((got == 9 || got == 10) && valid) {
       c.ks = splitk_rule(k.M, k.N, k.K, k.nbatch);   // the split is never tuned
       g_tuned[k] = c;
     }
@@ -168,7 +177,7 @@ static void record_tuned(const Key& k, const Cfg& c) {
   if (!path) return;
   FILE* fp = std::fopen(path, "a");
   if (!fp) return;
-  std::fprintf(fp, "%d %d %d %d %d %d %d %d %d %d\n", k.type, k.M, k.N, k.K, k.nbatch, k.flags, c.bm, c.bk,
+  std::fprintf(fp, "%d %d %d %d %d %d %d %d %d %d\n", k.type, k.M, k.N, k.K, k.nbatch, k.flags, c.bm, 16,
                c.ks, c.bn);
   std::fclose(fp);
 }
@@ -195,51 +204,83 @@ static int splitk_rule(int M, int N, int K, int nbatch) {
   return ks;
 }
 
-static Cfg heuristic(int M, int N, int K, int nbatch) {
-  const int64_t cus = 256;
-  const int ks = splitk_rule(M, N, K, nbatch);
-  int64_t t64 = ceil_div(M, 64) * ceil_div(N, 64) * (int64_t)nbatch;
-  if (t64 >= cus / 2) return {64, 16, ks};
-  return {32, 16, ks};
+// Estimated cost of a tile shape: rounds of work-groups over the 256 CUs
+// times a work-group's matrix-core time at its rate.  A work-group of one
+// wave shares its CU with three others.
+static double tile_cost(const Tile& t, int M, int N, int nbatch, int ks) {
+  const int64_t wgs = ceil_div(M, t.bm) * ceil_div(N, t.bn) * nbatch * ks;
+  const int64_t percu = t.threads == 64 ? 4 : 1;
+  const double rounds = (double)ceil_div(wgs, 256 * percu);
+  return rounds * percu * t.bm * t.bn / t.rate;
 }
 
-template <typename T, bool CT>
-static void launch_tiles(const GemmOp<T>& op, const Cfg& c, dim3 grid, hipStream_t st) {
-  if (cfg_bn(c) == 16 && c.bk == 16)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, 16, 1, CT>), grid, dim3(64), 0, st, op);
-  else if (cfg_bn(c) == 16 && c.bk == 32)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, 32, 1, CT>), grid, dim3(64), 0, st, op);
-  else if (cfg_bn(c) == 16)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, 64, 1, CT>), grid, dim3(64), 0, st, op);
-  else if (cfg_bn(c) == 80 && c.bk == 16)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 80, 16, 4, CT, 4>), grid, dim3(256), 0, st, op);
-  else if (cfg_bn(c) == 80)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 80, 32, 4, CT, 4>), grid, dim3(256), 0, st, op);
-  else if (c.bm == 64 && c.bk == 16)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 16, 4, CT>), grid, dim3(256), 0, st, op);
-  else if (c.bm == 64 && c.bk == 32)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 32, 4, CT>), grid, dim3(256), 0, st, op);
-  else if (c.bm == 64)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 64, 4, CT>), grid, dim3(256), 0, st, op);
-  else if (c.bk == 16)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, 16, 1, CT>), grid, dim3(64), 0, st, op);
-  else if (c.bk == 32)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, 32, 1, CT>), grid, dim3(64), 0, st, op);
-  else
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, 64, 1, CT>), grid, dim3(64), 0, st, op);
+static Cfg heuristic(int M, int N, int K, int nbatch) {
+  const int ks = splitk_rule(M, N, K, nbatch);
+  const Tile* best = nullptr;
+  double cost = 0.0;
+  for (const Tile& t : kTiles) {
+    const double c = tile_cost(t, M, N, nbatch, ks);
+    if (!best || c < cost) { best = &t; cost = c; }
+  }
+  return {best->bm, best->bn, ks};
+}
+
+template <typename T, bool CT, bool VEC>
+static void launch_tiles(const GemmOp<T>& op, const Cfg& c, hipStream_t st) {
+  const unsigned wgs = (unsigned)(ceil_div(op.M, c.bm) * ceil_div(op.N, c.bn) * op.nbatch * op.ksplit);
+  // K chunk: 16 for f64, 32 for f32 (a 16-byte load covers four k); the
+  // small tiles, latency-bound on each chunk, take twice as much
+  constexpr int BK = sizeof(T) == 8 ? 16 : 32, BK1 = VEC ? 2 * BK : BK;
+  switch (1000 * c.bm + c.bn) {
+    case 128064:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 64, BK, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      break;
+    case 64096:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 96, BK, 4, 2, CT, VEC>), dim3(wgs), dim3(512), 0, st, op);
+      break;
+    case 64080:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 80, BK, 4, 1, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      break;
+    case 64064:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, BK, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      break;
+    case 64032:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 32, BK, 4, 1, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      break;
+    case 32032:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, BK1, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      break;
+    default:
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, BK1, 1, 1, CT, VEC>), dim3(wgs), dim3(64), 0, st, op);
+      break;
+  }
+}
+
+// Whether an operand (rows x K, strides s_row, s_k, batch strides) can be
+// read 16 bytes at a time along its contiguous direction: pointer, other
+// strides and the extent of that direction all whole multiples of 16 bytes,
+// and a tile's offsets (at most 128 rows or 64 of k) below 2^32 bytes.
+template <typename T>
+static bool operand_aligned(const T* p, int64_t s_row, int64_t s_k, int64_t sb0, int64_t sb1, int rows, int K) {
+  constexpr int V = 16 / (int)sizeof(T);
+  if ((reinterpret_cast<uintptr_t>(p) & 15) != 0 || sb0 % V != 0 || sb1 % V != 0) return false;
+  const int64_t reach = (int64_t)1 << 22;   // elements: 127 rows of it are below 2^32 bytes
+  if (s_row == 1) return s_k % V == 0 && rows % V == 0 && s_k > 0 && s_k < reach;
+  return s_k == 1 && s_row % V == 0 && K % V == 0 && s_row > 0 && s_row < reach;
 }
 
 template <typename T>
 static void launch_cfg(GemmOp<T> op, const Cfg& c, hipStream_t st) {
   op.ksplit = c.ks;
-  int64_t tiles = ceil_div(op.M, c.bm) * ceil_div(op.N, cfg_bn(c));
-  dim3 grid((unsigned)tiles, (unsigned)op.nbatch, (unsigned)op.ksplit);
+  const bool vec = operand_aligned(op.A, op.sAi, op.sAk, op.sAb0, op.sAb1, op.M, op.K) &&
+                   operand_aligned(op.B, op.sBj, op.sBk, op.sBb0, op.sBb1, op.N, op.K);
   // column-contiguous outputs (and the column-major split-K slices) take the
   // swapped-fragment variant, whose lanes store consecutive rows
-  if (op.ksplit > 1 || op.sCi == 1)
-    launch_tiles<T, true>(op, c, grid, st);
-  else
-    launch_tiles<T, false>(op, c, grid, st);
+  const bool ct = op.ksplit > 1 || op.sCi == 1;
+  if (ct && vec) launch_tiles<T, true, true>(op, c, st);
+  else if (ct) launch_tiles<T, true, false>(op, c, st);
+  else if (vec) launch_tiles<T, false, true>(op, c, st);
+  else launch_tiles<T, false, false>(op, c, st);
   TTF_HIP(hipGetLastError());
   if (op.ksplit > 1) {
     int64_t total = (int64_t)op.M * op.N * op.nbatch;
@@ -255,26 +296,20 @@ static T* splitk_work(const GemmOp<T>& op, int ks) {
   return (T*)arena(kArenaSplitK, need);
 }
 
-// Times each candidate tile shape and K chunk twice with events and keeps
-// the fastest; the split-K factor is fixed by splitk_rule.  Only products that overwrite C (beta == 0) are tuned, since the
-// candidates run the product several times.
+// Times the three tile shapes that tile_cost ranks first twice with events
+// and keeps the fastest; the split-K factor is fixed by splitk_rule.  Only
+// products that overwrite C (beta == 0) are tuned, since the candidates run
+// the product several times.
 template <typename T>
 static Cfg tune(const GemmOp<T>& op0, hipStream_t st) {
+  const int ks = splitk_rule(op0.M, op0.N, op0.K, op0.nbatch);
+  std::vector<std::pair<double, Cfg>> ranked;
+  for (const Tile& t : kTiles)
+    ranked.push_back({tile_cost(t, op0.M, op0.N, op0.nbatch, ks), Cfg{t.bm, t.bn, ks}});
+  std::stable_sort(ranked.begin(), ranked.end(),
+                   [](const std::pair<double, Cfg>& x, const std::pair<double, Cfg>& y) { return x.first < y.first; });
   std::vector<Cfg> cands;
-  // square tiles, 64 x 80 tiles (four waves of 16 x 80) when N takes them
-  // evenly: N = 640 (a bond of 128 x MPO rank 5) splits into 8 such columns,
-  // so that a batch of 8 fills the 256 CUs once; and one-wave 32 x 16 tiles
-  // for N <= 16 (a block of search directions), which waste half as many
-  // matrix-core products on padding columns as 32 x 32
-  for (int bn : {0, 80, 16})
-    for (int bm : {64, 32})
-      for (int bk : {16, 32, 64}) {
-        if (bn == 80 && (bm != 64 || bk > 32 || op0.N % 80 != 0)) continue;
-        if (bn == 16 && (bm != 32 || op0.N > 16)) continue;
-        Cfg c{bm, bk, splitk_rule(op0.M, op0.N, op0.K, op0.nbatch)};
-        c.bn = bn;
-        cands.push_back(c);
-      }
+  for (size_t i = 0; i < ranked.size() && i < 3; ++i) cands.push_back(ranked[i].second);
   hipEvent_t e0, e1;
   TTF_HIP(hipEventCreate(&e0));
   TTF_HIP(hipEventCreate(&e1));
@@ -400,13 +435,13 @@ static void zgemm_launch_t(ZGemmOpT<R> op, hipStream_t st) {
   if (op.M <= 0 || op.N <= 0 || op.nbatch <= 0) return;
   if (op.nb0 <= 0) op.nb0 = 1;
   TTF_REQUIRE(op.nbatch <= 65535, "zgemm: batch count %d exceeds the grid limit", op.nbatch);
-  Cfg c = heuristic(op.M, op.N, op.K, op.nbatch);
-  int64_t tiles = ceil_div(op.M, c.bm) * ceil_div(op.N, c.bm);
+  const int bm = ceil_div(op.M, 64) * ceil_div(op.N, 64) * (int64_t)op.nbatch >= 128 ? 64 : 32;
+  int64_t tiles = ceil_div(op.M, bm) * ceil_div(op.N, bm);
   // few work-groups with a long K: slices of K in parallel (at least 48 deep
   // each), summed by a second launch
   op.ksplit = 1;
   op.work = nullptr;
-  if (c.bm == 32 && tiles * op.nbatch < 32 && op.K >= 128) {
+  if (bm == 32 && tiles * op.nbatch < 32 && op.K >= 128) {
     const int ks = (int)std::min<int64_t>({8, op.K / 48, ceil_div(64, tiles * op.nbatch)});
     if (ks > 1) {
       op.ksplit = ks;
@@ -416,7 +451,7 @@ static void zgemm_launch_t(ZGemmOpT<R> op, hipStream_t st) {
   dim3 grid((unsigned)tiles, (unsigned)op.nbatch, (unsigned)op.ksplit);
   // 32x32 tiles come with few work-groups, each one's K loop latency-bound
   // on its global loads: a 32-deep K chunk halves the trips
-  if (c.bm == 64)
+  if (bm == 64)
     hipLaunchKernelGGL((zgemm_mfma_kernel<R, 64, 64>), grid, dim3(256), 0, st, op);
   else if (op.K > 16)
     hipLaunchKernelGGL((zgemm_mfma_kernel<R, 32, 32, 32>), grid, dim3(256), 0, st, op);

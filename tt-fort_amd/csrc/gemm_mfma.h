@@ -9,12 +9,11 @@
 // b -> (b % nb0, b / nb0), each with its own stride, which covers "one GEMM
 // per vector of a block" and "one GEMM per bond index" at once.
 //
-// Tiling: 256 threads = 4 wave64s arranged 2x2; each wave owns a
-// (BM/2)x(BN/2) sub-tile made of 16x16 MFMA fragments
-// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).  K advances in chunks of
-// 16 staged through LDS; the next chunk is prefetched into registers while
-// the current one is consumed.  The global->LDS loader picks the coalesced
-// index order from the operand strides.  Work-group ids are remapped so that
+// Tiling: each wave of a work-group owns a sub-tile of 16x16 MFMA fragments
+// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).  K advances in chunks
+// staged through two LDS buffers; the next chunk is loaded while the current
+// one is consumed.  The global->LDS loader picks the coalesced index order
+// from the operand strides.  Work-group ids are remapped so that
 // neighbouring output tiles land on the same XCD (L2) of the 8-XCD chip.
 //
 // Split-K: with ksplit > 1 each work-group reduces a K range into a
@@ -77,85 +76,177 @@ __device__ __forceinline__ int xcd_remap(int wg, int total) {
   return (wg % nx) * per + (wg / nx);
 }
 
-// NW waves per work-group: NW = 4 arranges them 2x2 over the tile, NW = 1
-// lets a single wave own the whole tile.  Every wave keeps at least four
-// independent 16x16 accumulator chains (a 32x32 wave tile), since dependent
-// f64 MFMAs issue back to back only when several chains interleave.
+// One output tile BM x BN per work-group of WR x WC waves; each wave owns a
+// (BM/WR) x (BN/WC) sub-tile of 16x16 fragments and advances K four at a
+// time.
+//
+// The product is bound by the matrix cores when its tiles keep both operand
+// streams in flight, so the loads carry no per-lane conditions: a row or
+// column past the edge reads the last valid one (its results are not
+// stored), and only the chunk that crosses the end of K takes a form of the
+// loader that clamps k and zeroes by a select afterwards.  A load under a
+// lane condition compiles to a branch with a full wait each.  Measured, whole
+// local matvecs: rank 512, n 2, MPO rank 5, 8 vectors, f64 983 -> 761 us
+// (44 -> 57 TFLOP/s; a large product reaches 72 here); rank 64, n 64,
+// operator rank 6, one vector 67.5 -> 52.5 us in f64 and 53.9 -> 41.8 us in
+// f32 at ranks 61 and 57.  The next chunk is loaded to registers while the current one
+// is multiplied out of one of two LDS buffers (one barrier per chunk).  With
+// VEC, operands move 16 bytes per lane along their contiguous direction (the
+// launcher checks the alignment of pointers, strides and extents).
+//
 // CT (column-contiguous output, op.sCi == 1): the fragments are multiplied
 // in swapped order, B^T A^T, so that each accumulator holds a tile of C^T:
 // lane l then owns row l%16 of the 16x16 block and consecutive lanes store
 // consecutive rows (contiguous in memory) instead of consecutive columns.
-template <typename T, int BM, int BN, int BK, int NW = 4, bool CT = false, int WROWS = 0>
-__global__ __launch_bounds__(64 * NW) void gemm_mfma_kernel(GemmOp<T> op) {
-  constexpr int NT = 64 * NW;
-  constexpr int PAD = 2;
-  // wave rows: 2 x 2 waves by default, WROWS x (NW / WROWS) when given
-  constexpr int WR = WROWS > 0 ? WROWS : ((NW == 4) ? 2 : 1);
-  constexpr int WC = NW / WR;             // wave columns
+template <typename T, int V> struct VecOf;
+template <> struct VecOf<double, 2> { typedef double type __attribute__((ext_vector_type(2))); };
+template <> struct VecOf<float, 4> { typedef float type __attribute__((ext_vector_type(4))); };
+template <typename T> struct VecOf<T, 1> { typedef T type __attribute__((ext_vector_type(1))); };
+
+// One operand's tile loader: R rows (or columns) x BK of k, V elements per
+// load along the contiguous direction (`along_k`: that direction is k).
+// Thread t takes the vectors t, t + NT, ...
+template <typename T, int R, int BK, int NT, int V>
+struct TileLoad {
+  typedef typename VecOf<T, V>::type vec_t;
+  static constexpr int TOTAL = R * BK / V;
+  static constexpr int L = (TOTAL + NT - 1) / NT;
+  static constexpr bool EVEN = TOTAL % NT == 0;
+  static constexpr int PAD = 16 / (int)sizeof(T);   // keeps 16-byte LDS rows
+
+  // With V > 1 (where the launcher has checked that they fit) each vector is
+  // at a 32-bit offset from a uniform base, so that moving to the next chunk
+  // costs no vector instructions; else it has a pointer of its own.
+  const T* base;
+  unsigned off[V > 1 ? L : 1];
+  const T* p[V > 1 ? 1 : L];
+  int lds[L];        // LDS positions, k * (R + PAD) + row
+  vec_t v[L];
+  int64_t step;      // advance per chunk
+  int64_t sk;
+  bool along_k;
+
+  __device__ __forceinline__ static void split(int e, bool ak, int* row, int* k) {
+    if (ak) { *k = (e % (BK / V)) * V; *row = e / (BK / V); }
+    else { *row = (e % (R / V)) * V; *k = e / (R / V); }
+    if (!EVEN && e >= TOTAL) { *row = 0; *k = 0; }
+  }
+
+  // row0: first row of the tile, rows: the operand's extent, k0: first k
+  __device__ __forceinline__ void init(const T* op, int64_t s_row, int64_t s_k, int row0, int rows, int k0) {
+    along_k = V > 1 ? s_row != 1 : (s_row != 1 && s_k == 1);
+    sk = s_k;
+    step = s_k * BK;
+    base = op + s_row * row0 + s_k * k0;
+    // rows is a multiple of V when the vector runs along the rows
+    const int last = (along_k ? rows - 1 : rows - V) - row0;
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      int row, k;
+      split(threadIdx.x + q * NT, along_k, &row, &k);
+      lds[q] = k * (R + PAD) + row;
+      if constexpr (V > 1) off[q] = (unsigned)(sizeof(T) * (s_row * min(row, last) + s_k * k));
+      else p[q] = base + s_row * min(row, last) + s_k * k;
+    }
+  }
+  __device__ __forceinline__ void load() {
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      if constexpr (V > 1) {
+        v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base) + off[q]);
+      } else {
+        v[q][0] = *p[q];
+        p[q] += step;
+      }
+    }
+    base += step;
+  }
+  // the chunk that crosses the end of K: `left` = valid k of the chunk
+  __device__ __forceinline__ void load_tail(int left) {
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      int row, k;
+      split(threadIdx.x + q * NT, along_k, &row, &k);
+      const int64_t back = sk * (min(k, along_k ? left - V : left - 1) - k);
+      if constexpr (V > 1)
+        v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base + back) + off[q]);
+      else
+        v[q][0] = p[q][back];
+    }
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      int row, k;
+      split(threadIdx.x + q * NT, along_k, &row, &k);
+#pragma unroll
+      for (int u = 0; u < V; ++u) v[q][u] = k < left ? v[q][u] : T(0);
+    }
+  }
+  __device__ __forceinline__ void store(T* s) const {
+    if (V > 1 && !along_k) {
+#pragma unroll
+      for (int q = 0; q < L; ++q)
+        if (EVEN || (int)threadIdx.x + q * NT < TOTAL) *reinterpret_cast<vec_t*>(s + lds[q]) = v[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < L; ++q)
+        if (EVEN || (int)threadIdx.x + q * NT < TOTAL) {
+#pragma unroll
+          for (int u = 0; u < V; ++u) s[lds[q] + u * (R + PAD)] = v[q][u];
+        }
+    }
+  }
+};
+
+//
+// The second launch bound (two waves per SIMD, so at most 256 registers)
+// keeps the accumulators in vector registers: without it the compiler puts
+// them in accumulation registers and copies them in and out on every turn of
+// the loop, which alone held f64 MFMA loops at 33 (one wave per SIMD) to 50
+// of the 69 to 77 TFLOP/s they reach here.
+template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op) {
+  constexpr int NT = 64 * WR * WC;
+  constexpr int V = VEC ? 16 / (int)sizeof(T) : 1;
   constexpr int WM = BM / WR, WN = BN / WC;
   constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int LA = BM * BK / NT;   // A elements per thread
-  constexpr int LB = BN * BK / NT;   // B elements per thread
+  static_assert(FM * 16 * WR == BM && FN * 16 * WC == BN, "wave tiles of whole fragments");
   typedef typename Acc4<T>::type acc_t;
+  typedef TileLoad<T, BM, BK, NT, V> LoadA;
+  typedef TileLoad<T, BN, BK, NT, V> LoadB;
+  constexpr int LDA = BM + LoadA::PAD, LDB = BN + LoadB::PAD;
+  static_assert(V == 1 || (LDA * sizeof(T) % 16 == 0 && LDB * sizeof(T) % 16 == 0), "LDS rows of whole 16 bytes");
 
-  __shared__ T As[BK][BM + PAD];
-  __shared__ T Bs[BK][BN + PAD];
+  __shared__ __attribute__((aligned(16))) T As[2][BK * LDA];
+  __shared__ __attribute__((aligned(16))) T Bs[2][BK * LDB];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WC, wn = wave % WC;
 
+  // consecutive logical tiles share an XCD and so an L2; they go down bands
+  // of eight tile rows, so that the tiles in flight on an XCD read about as
+  // many rows of A as columns of B
   const int tilesM = (op.M + BM - 1) / BM;
   const int tilesN = (op.N + BN - 1) / BN;
   const int ntiles = tilesM * tilesN;
-  const int tile = xcd_remap(blockIdx.x, ntiles);
-  const int tm = tile / tilesN, tn = tile % tilesN;
-
-  const int b = blockIdx.y;
-  const int b0 = b % op.nb0, b1 = b / op.nb0;
-  const T* __restrict__ A = op.A + b0 * op.sAb0 + b1 * op.sAb1;
-  const T* __restrict__ B = op.B + b0 * op.sBb0 + b1 * op.sBb1;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int z = wg / (ntiles * op.nbatch);
+  const int wr = wg - z * (ntiles * op.nbatch);
+  const int b = wr / ntiles, tile = wr - b * ntiles;
+  const int band = tile / (8 * tilesN), inb = tile - band * (8 * tilesN);
+  const int bandM = min(8, tilesM - 8 * band);
+  const int tn = inb / bandM, tm = 8 * band + inb - tn * bandM;
+  const int b1 = b / op.nb0, b0 = b - b1 * op.nb0;
 
   // K range of this work-group.  Split-K ranges are multiples of 64 for every
   // BK, so the slices (and the order of the sums) depend on ksplit alone.
   constexpr int KG = 64;
   static_assert(KG % BK == 0, "split-K granularity must be a multiple of BK");
-  const int kchunk = op.ksplit > 1 ? ((op.K + op.ksplit - 1) / op.ksplit + KG - 1) / KG * KG
-                                   : ((op.K + BK - 1) / BK) * BK;
-  const int kbeg = blockIdx.z * kchunk;
+  const int kchunk = op.ksplit > 1 ? ((op.K + op.ksplit - 1) / op.ksplit + KG - 1) / KG * KG : op.K;
+  const int kbeg = z * kchunk;
   const int kend = min(op.K, kbeg + kchunk);
-
-  const bool a_ifast = (op.sAi == 1);
-  const bool b_jfast = (op.sBj == 1);
-
-  T ra[LA], rb[LB];
-  int ai[LA], ak[LA], bk[LB], bj[LB];
-#pragma unroll
-  for (int q = 0; q < LA; ++q) {
-    int idx = tid + q * NT;
-    if (a_ifast) { ai[q] = idx % BM; ak[q] = idx / BM; }
-    else         { ak[q] = idx % BK; ai[q] = idx / BK; }
-  }
-#pragma unroll
-  for (int q = 0; q < LB; ++q) {
-    int idx = tid + q * NT;
-    if (b_jfast) { bj[q] = idx % BN; bk[q] = idx / BN; }
-    else         { bk[q] = idx % BK; bj[q] = idx / BK; }
-  }
-
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < LA; ++q) {
-      int gi = tm * BM + ai[q], gk = k0 + ak[q];
-      ra[q] = (gi < op.M && gk < kend) ? A[gi * op.sAi + gk * op.sAk] : T(0);
-    }
-#pragma unroll
-    for (int q = 0; q < LB; ++q) {
-      int gj = tn * BN + bj[q], gk = k0 + bk[q];
-      rb[q] = (gj < op.N && gk < kend) ? B[gk * op.sBk + gj * op.sBj] : T(0);
-    }
-  };
+  const int nch = (kend - kbeg + BK - 1) / BK;   // <= 0 for an empty range
 
   acc_t acc[FM][FN];
 #pragma unroll
@@ -163,28 +254,54 @@ __global__ __launch_bounds__(64 * NW) void gemm_mfma_kernel(GemmOp<T> op) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
-  if (kbeg < kend) load(kbeg);
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
+  if (nch > 0) {   // uniform
+    LoadA la;
+    LoadB lb;
+    la.init(op.A + b0 * op.sAb0 + b1 * op.sAb1, op.sAi, op.sAk, tm * BM, op.M, kbeg);
+    lb.init(op.B + b0 * op.sBb0 + b1 * op.sBb1, op.sBj, op.sBk, tn * BN, op.N, kbeg);
+    auto load = [&](int c) {
+      const int left = kend - kbeg - c * BK;
+      if (left >= BK) {
+        la.load();
+        lb.load();
+      } else {
+        la.load_tail(left);
+        lb.load_tail(left);
+      }
+    };
+    const int arow = (lane >> 4) * LDA + wm * WM + (lane & 15);
+    const int brow = (lane >> 4) * LDB + wn * WN + (lane & 15);
+    auto multiply = [&](int buf) {
+      const T* as = As[buf] + arow;
+      const T* bs = Bs[buf] + brow;
+#pragma unroll
+      for (int kk = 0; kk < BK; kk += 4) {
+        T af[FM], bf[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) af[i] = as[kk * LDA + i * 16];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bf[j] = bs[kk * LDB + j * 16];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = CT ? mfma16(bf[j], af[i], acc[i][j]) : mfma16(af[i], bf[j], acc[i][j]);
+      }
+    };
+    load(0);
+    la.store(As[0]);
+    lb.store(Bs[0]);
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < LA; ++q) As[ak[q]][ai[q]] = ra[q];
-#pragma unroll
-    for (int q = 0; q < LB; ++q) Bs[bk[q]][bj[q]] = rb[q];
-    __syncthreads();
-    if (k0 + BK < kend) load(k0 + BK);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T af[FM], bf[FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = As[kk + (lane >> 4)][wm * WM + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = Bs[kk + (lane >> 4)][wn * WN + j * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = CT ? mfma16(bf[j], af[i], acc[i][j]) : mfma16(af[i], bf[j], acc[i][j]);
+    // one exit, after the last chunk but one: a second way out of the loop
+    // makes the compiler copy every accumulator in each turn
+    for (int c = 0; c < nch - 1; ++c) {
+      load(c + 1);
+      multiply(c & 1);
+      la.store(As[(c + 1) & 1]);
+      lb.store(Bs[(c + 1) & 1]);
+      __syncthreads();
     }
+    multiply((nch - 1) & 1);
   }
 
   // Epilogue: lane l, register r holds row mfma_row<T>(l, r), column l%16
@@ -226,7 +343,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_mfma_kernel(GemmOp<T> op) {
           }
         }
   } else {
-    T* __restrict__ W = op.work + ((int64_t)blockIdx.z * op.nbatch + b) * op.M * op.N;
+    T* __restrict__ W = op.work + ((int64_t)z * op.nbatch + b) * op.M * op.N;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -521,11 +638,10 @@ __global__ void zgemm_splitk_reduce(ZGemmOpT<R> op) {
 }
 
 // ---------------------------------------------------------------- launchers
-// Implemented in gemm.hip.  The tile shape (64x64 or 32x32, K chunk 16 or
-// 32) and the split-K factor of each GEMM are chosen by a runtime autotuner
-// keyed on (type, M, N, K, batch, operand layout): the first launch of a new
-// shape times the candidates with events on the stream and caches the
-// fastest.  Small-panel products (K <= 64, N <= 32, B shared by all batches)
+// Implemented in gemm.hip.  The tile shape of each GEMM is chosen by a
+// runtime autotuner keyed on (type, M, N, K, batch, operand layout): the
+// first launch of a new shape times the few tiles that a fill model ranks
+// first with events on the stream and caches the fastest.  Small-panel products (K <= 64, N <= 32, B shared by all batches)
 // go to a dedicated vector kernel instead of the matrix cores.
 template <typename T>
 void gemm_launch(GemmOp<T> op, hipStream_t st);

@@ -26,7 +26,7 @@ constexpr int kTsgRows = 64;   // rows per chunk: one per lane of a wave
 // partials of one output, one batch of loads each, and a row sum combines
 // them.  X's columns may come from two matrices: columns [0, p1) from X,
 // the rest from X2 (ld ldx2).
-__global__ __launch_bounds__(256) void tsgram_partial(int N, int p, int q, const double* __restrict__ X,
+__global__ __launch_bounds__(256, 2) void tsgram_partial(int N, int p, int q, const double* __restrict__ X,
                                                       int64_t ldx, int p1, const double* __restrict__ X2,
                                                       int64_t ldx2, const double* __restrict__ Y,
                                                       int64_t ldy, double* __restrict__ part) {
