@@ -203,27 +203,116 @@ struct TileLoad {
 // them in accumulation registers and copies them in and out on every turn of
 // the loop, which alone held f64 MFMA loops at 33 (one wave per SIMD) to 50
 // of the 69 to 77 TFLOP/s they reach here.
-template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC>
-__global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op) {
-  constexpr int NT = 64 * WR * WC;
-  constexpr int V = VEC ? 16 / (int)sizeof(T) : 1;
-  constexpr int WM = BM / WR, WN = BN / WC;
-  constexpr int FM = WM / 16, FN = WN / 16;
+// GemmTile holds one work-group's tile: sums() computes the tile at (row0,
+// col0) over k in [kbeg, kend), after which acc[i][j][r] is the sum of row
+// row0 + row(i, r) and column col0 + col(j, r) (either may lie past the
+// operand's extent).  With FOLD each chunk's products are summed by
+// themselves and then added, which shortens the rounding chain of long f32
+// sums.
+template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC, bool FOLD = false>
+struct GemmTile {
+  static constexpr int NT = 64 * WR * WC;
+  static constexpr int V = VEC ? 16 / (int)sizeof(T) : 1;
+  static constexpr int WM = BM / WR, WN = BN / WC;
+  static constexpr int FM = WM / 16, FN = WN / 16;
   static_assert(FM * 16 * WR == BM && FN * 16 * WC == BN, "wave tiles of whole fragments");
   typedef typename Acc4<T>::type acc_t;
   typedef TileLoad<T, BM, BK, NT, V> LoadA;
   typedef TileLoad<T, BN, BK, NT, V> LoadB;
-  constexpr int LDA = BM + LoadA::PAD, LDB = BN + LoadB::PAD;
+  static constexpr int LDA = BM + LoadA::PAD, LDB = BN + LoadB::PAD;
   static_assert(V == 1 || (LDA * sizeof(T) % 16 == 0 && LDB * sizeof(T) % 16 == 0), "LDS rows of whole 16 bytes");
 
-  __shared__ __attribute__((aligned(16))) T As[2][BK * LDA];
-  __shared__ __attribute__((aligned(16))) T Bs[2][BK * LDB];
+  acc_t acc[FM][FN];
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / WC, wn = wave % WC;
+  __device__ __forceinline__ static int row(int i, int r) {
+    const int lane = threadIdx.x & 63;
+    return (int)(threadIdx.x >> 6) / WC * WM + i * 16 + (CT ? (lane & 15) : mfma_row<T>(lane, r));
+  }
+  __device__ __forceinline__ static int col(int j, int r) {
+    const int lane = threadIdx.x & 63;
+    return (int)(threadIdx.x >> 6) % WC * WN + j * 16 + (CT ? mfma_row<T>(lane, r) : (lane & 15));
+  }
 
+  __device__ __forceinline__ void sums(const GemmOp<T>& op, const T* A, const T* B, int row0, int col0, int kbeg,
+                                       int kend) {
+    __shared__ __attribute__((aligned(16))) T As[2][BK * LDA];
+    __shared__ __attribute__((aligned(16))) T Bs[2][BK * LDB];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave / WC, wn = wave % WC;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    const int nch = (kend - kbeg + BK - 1) / BK;   // <= 0 for an empty range
+    if (nch <= 0) return;                          // uniform
+    LoadA la;
+    LoadB lb;
+    la.init(A, op.sAi, op.sAk, row0, op.M, kbeg);
+    lb.init(B, op.sBj, op.sBk, col0, op.N, kbeg);
+    auto load = [&](int c) {
+      const int left = kend - kbeg - c * BK;
+      if (left >= BK) {
+        la.load();
+        lb.load();
+      } else {
+        la.load_tail(left);
+        lb.load_tail(left);
+      }
+    };
+    const int arow = (lane >> 4) * LDA + wm * WM + (lane & 15);
+    const int brow = (lane >> 4) * LDB + wn * WN + (lane & 15);
+    auto multiply = [&](int buf) {
+      const T* as = As[buf] + arow;
+      const T* bs = Bs[buf] + brow;
+      acc_t own[FM][FN];
+      auto& sum = FOLD ? own : acc;
+      if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) own[i][j] = acc_t{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int kk = 0; kk < BK; kk += 4) {
+        T af[FM], bf[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) af[i] = as[kk * LDA + i * 16];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bf[j] = bs[kk * LDB + j * 16];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            sum[i][j] = CT ? mfma16(bf[j], af[i], sum[i][j]) : mfma16(af[i], bf[j], sum[i][j]);
+      }
+      if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] += own[i][j];
+      }
+    };
+    load(0);
+    la.store(As[0]);
+    lb.store(Bs[0]);
+    __syncthreads();
+    // one exit, after the last chunk but one: a second way out of the loop
+    // makes the compiler copy every accumulator in each turn
+    for (int c = 0; c < nch - 1; ++c) {
+      load(c + 1);
+      multiply(c & 1);
+      la.store(As[(c + 1) & 1]);
+      lb.store(Bs[(c + 1) & 1]);
+      __syncthreads();
+    }
+    multiply((nch - 1) & 1);
+  }
+};
+
+template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op) {
+  typedef GemmTile<T, BM, BN, BK, WR, WC, CT, VEC> Tile;
+  constexpr int FM = Tile::FM, FN = Tile::FN;
   // consecutive logical tiles share an XCD and so an L2; they go down bands
   // of eight tile rows, so that the tiles in flight on an XCD read about as
   // many rows of A as columns of B
@@ -246,66 +335,10 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op
   const int kchunk = op.ksplit > 1 ? ((op.K + op.ksplit - 1) / op.ksplit + KG - 1) / KG * KG : op.K;
   const int kbeg = z * kchunk;
   const int kend = min(op.K, kbeg + kchunk);
-  const int nch = (kend - kbeg + BK - 1) / BK;   // <= 0 for an empty range
 
-  acc_t acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  Tile t;
+  t.sums(op, op.A + b0 * op.sAb0 + b1 * op.sAb1, op.B + b0 * op.sBb0 + b1 * op.sBb1, tm * BM, tn * BN, kbeg, kend);
 
-  if (nch > 0) {   // uniform
-    LoadA la;
-    LoadB lb;
-    la.init(op.A + b0 * op.sAb0 + b1 * op.sAb1, op.sAi, op.sAk, tm * BM, op.M, kbeg);
-    lb.init(op.B + b0 * op.sBb0 + b1 * op.sBb1, op.sBj, op.sBk, tn * BN, op.N, kbeg);
-    auto load = [&](int c) {
-      const int left = kend - kbeg - c * BK;
-      if (left >= BK) {
-        la.load();
-        lb.load();
-      } else {
-        la.load_tail(left);
-        lb.load_tail(left);
-      }
-    };
-    const int arow = (lane >> 4) * LDA + wm * WM + (lane & 15);
-    const int brow = (lane >> 4) * LDB + wn * WN + (lane & 15);
-    auto multiply = [&](int buf) {
-      const T* as = As[buf] + arow;
-      const T* bs = Bs[buf] + brow;
-#pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        T af[FM], bf[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) af[i] = as[kk * LDA + i * 16];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) bf[j] = bs[kk * LDB + j * 16];
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = CT ? mfma16(bf[j], af[i], acc[i][j]) : mfma16(af[i], bf[j], acc[i][j]);
-      }
-    };
-    load(0);
-    la.store(As[0]);
-    lb.store(Bs[0]);
-    __syncthreads();
-    // one exit, after the last chunk but one: a second way out of the loop
-    // makes the compiler copy every accumulator in each turn
-    for (int c = 0; c < nch - 1; ++c) {
-      load(c + 1);
-      multiply(c & 1);
-      la.store(As[(c + 1) & 1]);
-      lb.store(Bs[(c + 1) & 1]);
-      __syncthreads();
-    }
-    multiply((nch - 1) & 1);
-  }
-
-  // Epilogue: lane l, register r holds row mfma_row<T>(l, r), column l%16
-  // of each 16x16 block (CT: row l%16, column mfma_row<T>(l, r)).
   if (op.ksplit == 1) {
     T* __restrict__ C = op.C + b0 * op.sCb0 + b1 * op.sCb1;
     // with beta != 0 the tile's C elements are all loaded (from clamped
@@ -319,10 +352,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op
         for (int j = 0; j < FN; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int fr = CT ? (lane & 15) : mfma_row<T>(lane, r);
-            const int fc = CT ? mfma_row<T>(lane, r) : (lane & 15);
-            const int gi = min(tm * BM + wm * WM + i * 16 + fr, op.M - 1);
-            const int gj = min(tn * BN + wn * WN + j * 16 + fc, op.N - 1);
+            const int gi = min(tm * BM + Tile::row(i, r), op.M - 1);
+            const int gj = min(tn * BN + Tile::col(j, r), op.N - 1);
             cv[i][j][r] = C[gi * op.sCi + gj * op.sCj];
           }
     }
@@ -332,12 +363,9 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int fr = CT ? (lane & 15) : mfma_row<T>(lane, r);
-          const int fc = CT ? mfma_row<T>(lane, r) : (lane & 15);
-          int gi = tm * BM + wm * WM + i * 16 + fr;
-          int gj = tn * BN + wn * WN + j * 16 + fc;
+          const int gi = tm * BM + Tile::row(i, r), gj = tn * BN + Tile::col(j, r);
           if (gi < op.M && gj < op.N) {
-            T v = op.alpha * acc[i][j][r];
+            T v = op.alpha * t.acc[i][j][r];
             if (op.beta != T(0)) v += op.beta * cv[i][j][r];
             C[gi * op.sCi + gj * op.sCj] = v;
           }
@@ -350,11 +378,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int fr = CT ? (lane & 15) : mfma_row<T>(lane, r);
-          const int fc = CT ? mfma_row<T>(lane, r) : (lane & 15);
-          int gi = tm * BM + wm * WM + i * 16 + fr;
-          int gj = tn * BN + wn * WN + j * 16 + fc;
-          if (gi < op.M && gj < op.N) W[gi + (int64_t)gj * op.M] = acc[i][j][r];
+          const int gi = tm * BM + Tile::row(i, r), gj = tn * BN + Tile::col(j, r);
+          if (gi < op.M && gj < op.N) W[gi + (int64_t)gj * op.M] = t.acc[i][j][r];
         }
   }
 }

@@ -125,91 +125,183 @@ __global__ __launch_bounds__(256) void features_kernel(int rx1, int n, int rx2, 
   }
 }
 
-// Y (N x M, ld N) = act(W^T X + b): W bf16 (K x N, ld K), X fp32 (K x M,
-// ld K).  Work-group tile 64 (N) x 64 (M), 4 waves of 32 x 32, K in chunks
-// of 16 through LDS; v_mfma_f32_16x16x4f32 with the weights widened on load.
-// With SKIP (the output layer), X0 are the network's input features and
-// Y(n, m) += X0(3 kMlpBlock + n, m) / X0(n, m): the point-Jacobi solution of
-// the block, which the layers correct.
-template <bool RELU, bool SKIP>
-__global__ __launch_bounds__(256) void layer_kernel(int M, int K, int N, const float* __restrict__ X,
-                                                    const uint16_t* __restrict__ W, const float* __restrict__ bias,
-                                                    float* __restrict__ Y, const float* __restrict__ X0) {
-  constexpr int BK = 16, PAD = 4;
-  __shared__ float Ws[BK][64 + PAD];
-  __shared__ float Xs[BK][64 + PAD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wn = wave & 1, wm = wave >> 1;
-  const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 64;
-  f4_t acc[2][2];
+// ---- training: the forward and backward products on the f32 matrix cores,
+// through the GEMM engine's tiles with the elementwise work in their
+// epilogues.  A batch of 1024 columns is a few tens of MFLOP, so what counts
+// is launches and how many work-groups each one has: seven launches of 32 x
+// 32 or 64 x 64 tiles, in place of seventeen whose bias sums ran one thread
+// per row.  Loss and gradient of 1024 columns: 873 -> 128 us, 52 us of it in
+// these kernels and the rest in bringing 0.6 MB of gradient to the host.
+//
+// Y (N x M, ld N) = act(W^T X + b) for W (K x N, ld K; the fp32 values of
+// the bf16 weights) and X (K x M, ld K).  MODE 0: act = ReLU, Y = H.  MODE 1
+// (the output layer): the point-Jacobi term X0(3 kMlpBlock + n, m) /
+// X0(n, m) of the input features X0 is added, Y = dL/dY = f (y - T) with the
+// targets T, and part[work-group] = the sum of (y - T)^2.
+typedef GemmTile<float, 32, 32, 64, 2, 2, true, true, true> LayerTile;
+
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void train_layer_kernel(GemmOp<float> op, const float* __restrict__ bias,
+                                                             const float* __restrict__ X0,
+                                                             const float* __restrict__ T, float f,
+                                                             double* __restrict__ part) {
+  const int tilesN = (op.N + 31) / 32;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int tm = wg / tilesN, tn = wg - tm * tilesN;
+  LayerTile t;
+  t.sums(op, op.A, op.B, tm * 32, tn * 32, 0, op.K);
+  // the epilogue's operands, from clamped in-range indices before any is
+  // used: loaded under each output's own condition they become a branch
+  // with a full wait apiece
+  float eb[4], ed[4], ex[4], et[4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int idx = tid + 256 * q;
-      const int kk = idx & (BK - 1), cc = idx >> 4;
-      const int gn = n0 + cc, gm = m0 + cc;
-      Ws[kk][cc] = gn < N ? from_bf16(W[(k0 + kk) + (int64_t)K * gn]) : 0.f;
-      Xs[kk][cc] = gm < M ? X[(k0 + kk) + (int64_t)K * gm] : 0.f;
+  for (int r = 0; r < 4; ++r) {
+    const int n = min(tm * 32 + LayerTile::row(0, r), op.M - 1);
+    const int m = min(tn * 32 + LayerTile::col(0, r), op.N - 1);
+    eb[r] = bias[n];
+    if (MODE == 1) {
+      ed[r] = X0[n + (int64_t)kMlpIn * m];
+      ex[r] = X0[3 * kMlpBlock + n + (int64_t)kMlpIn * m];
+      et[r] = T[n + (int64_t)op.M * m];
     }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = Ws[kk + (lane >> 4)][wn * 32 + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = Xs[kk + (lane >> 4)][wm * 32 + j * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
   }
-  // the epilogue's operands for the 16 outputs (bias, and with SKIP the
-  // block diagonal and the residual), loaded from clamped in-range indices
-  // before any is used: loaded under each output's own condition they
-  // become a branch with a full wait apiece
-  float eb[16], ed[16], ex[16];
+  double s = 0.0;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int q = i * 8 + j * 4 + r;
-        const int gn = min(n0 + wn * 32 + i * 16 + mfma_row<float>(lane, r), N - 1);
-        const int gm = min(m0 + wm * 32 + j * 16 + (lane & 15), M - 1);
-        eb[q] = bias[gn];
-        if (SKIP) {
-          ed[q] = X0[gn + (int64_t)kMlpIn * gm];
-          ex[q] = X0[3 * kMlpBlock + gn + (int64_t)kMlpIn * gm];
-        }
+  for (int r = 0; r < 4; ++r) {
+    const int n = tm * 32 + LayerTile::row(0, r), m = tn * 32 + LayerTile::col(0, r);
+    if (n < op.M && m < op.N) {
+      float val = t.acc[0][0][r] + eb[r];
+      if (MODE == 0) {
+        val = fmaxf(val, 0.f);
+      } else {
+        val += ed[r] != 0.f ? ex[r] / ed[r] : 0.f;
+        const float d = val - et[r];
+        s += (double)d * d;
+        val = f * d;
       }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int q = i * 8 + j * 4 + r;
-        const int gn = n0 + wn * 32 + i * 16 + mfma_row<float>(lane, r);
-        const int gm = m0 + wm * 32 + j * 16 + (lane & 15);
-        if (gn < N && gm < M) {
-          float val = acc[i][j][r] + eb[q];
-          if (RELU) val = fmaxf(val, 0.f);
-          if (SKIP) val += ed[q] != 0.f ? ex[q] / ed[q] : 0.f;
-          Y[gn + (int64_t)N * gm] = val;
-        }
-      }
+      op.C[n + (int64_t)op.M * m] = val;
+    }
+  }
+  if (MODE == 1) {
+    __shared__ double red[4];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  }
 }
 
-// The inference form of layer_kernel on gfx950's bf16 matrix cores: the
-// same Y = act(W^T X + b) (+ the point-Jacobi term with SKIP), with the
+// dH (kMlpHid x M) = W D with the ReLU derivative from the activation H
+// itself: zero where H is not positive.
+__global__ __launch_bounds__(256, 2) void train_back_kernel(GemmOp<float> op, const float* __restrict__ H) {
+  const int tilesN = (op.N + 31) / 32;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int tm = wg / tilesN, tn = wg - tm * tilesN;
+  LayerTile t;
+  t.sums(op, op.A, op.B, tm * 32, tn * 32, 0, op.K);
+  float h[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    h[r] = H[min(tm * 32 + LayerTile::row(0, r), op.M - 1) +
+             (int64_t)op.M * min(tn * 32 + LayerTile::col(0, r), op.N - 1)];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int n = tm * 32 + LayerTile::row(0, r), m = tn * 32 + LayerTile::col(0, r);
+    if (n < op.M && m < op.N) op.C[n + (int64_t)op.M * m] = h[r] > 0.f ? t.acc[0][0][r] : 0.f;
+  }
+}
+
+// All gradients over one slice of columns per group of work-groups, into
+// the slice's own parameter vector part + slice kMlpParams: the tiles of the
+// three weight gradients In_l D_l^T (64 x 64, four rows of tiles each), then
+// the bias gradients, 64 rows of D_l per work-group.
+constexpr int kGradSlices = 16;
+constexpr int kGradTiles = 4 * (kMlpHid + kMlpHid + kMlpOut) / 64;   // 36 weight tiles
+constexpr int kGradRows = (kMlpHid + kMlpHid + kMlpOut) / 64;        // 9 bias groups
+static_assert(kMlpIn == 256 && kMlpHid == 256 && kMlpOut == 64, "gradient tiles");
+typedef GemmTile<float, 64, 64, 32, 2, 2, true, true, true> GradTile;
+
+struct WeightGrads {
+  const float* in[3];   // X, H1, H2 (256 x M)
+  const float* d[3];    // dH1, dH2, dY (256, 256, 64 rows x M)
+  int M, slice, nslices;
+};
+
+__global__ __launch_bounds__(256, 2) void weight_grad_kernel(WeightGrads a, float* __restrict__ part) {
+  const int per = kGradTiles + kGradRows;
+  const int s = blockIdx.x / per;
+  int u = blockIdx.x - s * per;
+  const int m0 = s * a.slice, m1 = min(a.M, m0 + a.slice);
+  float* out = part + (int64_t)kMlpParams * s;
+  const bool weight = u < kGradTiles;
+  if (!weight) u = 4 * (u - kGradTiles);
+  const int l = u < 16 ? 0 : (u < 32 ? 1 : 2);   // 16, 16 and 4 tiles
+  u -= 16 * l;
+  const int tn = u >> 2, tm = u & 3, cols = l == 2 ? kMlpOut : kMlpHid;
+  const float* D = a.d[l];
+  if (weight) {
+    out += l == 0 ? kMlpOffW1 : (l == 1 ? kMlpOffW2 : kMlpOffW3);
+    GemmOp<float> op{};
+    op.M = kMlpIn; op.N = cols; op.K = a.M;
+    op.sAi = 1; op.sAk = kMlpIn;
+    op.sBj = 1; op.sBk = cols;
+    GradTile t;
+    t.sums(op, a.in[l], D, 64 * tm, 64 * tn, m0, m1);
+#pragma unroll
+    for (int i = 0; i < GradTile::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < GradTile::FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          out[64 * tm + GradTile::row(i, r) + kMlpIn * (64 * tn + GradTile::col(j, r))] = t.acc[i][j][r];
+  } else {
+    __shared__ float red[4][64];
+    const int r = threadIdx.x & 63, g = threadIdx.x >> 6, row = 64 * tn + r;
+    float sum = 0.f;
+    for (int m = m0 + g; m < m1; m += 32) {   // eight columns of this thread in flight
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = D[row + (int64_t)cols * min(m + 4 * q, m1 - 1)];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sum += m + 4 * q < m1 ? v[q] : 0.f;
+    }
+    red[g][r] = sum;
+    __syncthreads();
+    if (g == 0)
+      out[(l == 0 ? kMlpOffB1 : (l == 1 ? kMlpOffB2 : kMlpOffB3)) + row] =
+          (red[0][r] + red[1][r]) + (red[2][r] + red[3][r]);
+  }
+}
+
+// g = the sum of the slices in order; the last work-group adds the loss
+// partials instead: loss = scale * their sum.
+__global__ __launch_bounds__(256) void grad_reduce_kernel(int nslices, const float* __restrict__ part,
+                                                          float* __restrict__ g, int nloss,
+                                                          const double* __restrict__ lpart, double scale,
+                                                          double* __restrict__ loss) {
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ double red[4];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < nloss; i += 256) s += lpart[i];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) *loss = ((red[0] + red[1]) + (red[2] + red[3])) * scale;
+    return;
+  }
+  const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (e >= kMlpParams) return;
+  float v[kGradSlices];
+#pragma unroll
+  for (int s = 0; s < kGradSlices; ++s) v[s] = part[e + kMlpParams * (int64_t)min(s, nslices - 1)];
+  float sum = 0.f;
+#pragma unroll
+  for (int s = 0; s < kGradSlices; ++s) sum += s < nslices ? v[s] : 0.f;
+  g[e] = sum;
+}
+
+// The inference form of the layers on gfx950's bf16 matrix cores: the same
+// Y = act(W^T X + b) (+ the point-Jacobi term with SKIP), with the
 // activations X rounded to bf16 (round to nearest even) and the products
 // accumulated in fp32 by v_mfma_f32_16x16x32_bf16.  K = 256 for every layer
 // of the network.  Lane l feeds row (or column) l % 16 and the eight
@@ -336,47 +428,6 @@ __global__ __launch_bounds__(256) void targets_kernel(int rx1, int n, int rx2, c
   T[lane + (int64_t)kMlpOut * col] = (float)(z[b1 + (int64_t)rx1 * (lane + (int64_t)n * b2)] * (double)inv[col]);
 }
 
-// dY = 2 (Y - T) / (M * Out) and per-work-group partial sums of (Y - T)^2
-__global__ __launch_bounds__(256) void loss_grad_kernel(int64_t count, int M, const float* __restrict__ Y,
-                                                        const float* __restrict__ T, float* __restrict__ dY,
-                                                        double* __restrict__ part) {
-  __shared__ double red[4];
-  double s = 0.0;
-  const float f = 2.0f / ((float)M * (float)kMlpOut);
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < count; e += (int64_t)gridDim.x * blockDim.x) {
-    const float d = Y[e] - T[e];
-    dY[e] = f * d;
-    s += (double)d * d;
-  }
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-__global__ void sum_partials_kernel(int np, const double* __restrict__ part, double scale, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < np; ++i) s += part[i];
-    *out = s * scale;
-  }
-}
-
-// dH *= (H > 0) (ReLU derivative from the activation itself)
-__global__ void relu_mask_kernel(int64_t count, const float* __restrict__ H, float* __restrict__ dH) {
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < count; e += (int64_t)gridDim.x * blockDim.x)
-    if (!(H[e] > 0.f)) dH[e] = 0.f;
-}
-
-// out(r) = sum_c D(r, c), D (rows x cols, ld rows); one thread per row
-__global__ void rowsum_kernel(int rows, int cols, const float* __restrict__ D, float* __restrict__ out) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  float s = 0.f;
-  for (int c = 0; c < cols; ++c) s += D[r + (int64_t)rows * c];
-  out[r] = s;
-}
-
 __global__ void gather_cols_kernel(int rows, int ncols, const int* __restrict__ idx, const float* __restrict__ src,
                                    float* __restrict__ dst) {
   const int64_t total = (int64_t)rows * ncols;
@@ -416,23 +467,6 @@ void features(int rx1, int n, int rx2, int ra1, int ra2, const double* phi1, con
 }
 
 template <bool RELU, bool SKIP>
-void layer(int M, int K, int N, const float* X, const uint16_t* W, const float* b, float* Y, const float* X0,
-           hipStream_t st) {
-  dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  hipLaunchKernelGGL((layer_kernel<RELU, SKIP>), grid, dim3(256), 0, st, M, K, N, X, W, b, Y, X0);
-  TTF_HIP(hipGetLastError());
-}
-
-// H1, H2 (Hid x M), Y (Out x M)
-void forward(int M, const float* X, float* H1, float* H2, float* Y, hipStream_t st) {
-  const uint16_t* w = g_model.wbf;
-  const float* p = g_model.master;
-  layer<true, false>(M, kMlpIn, kMlpHid, X, w + kMlpOffW1, p + kMlpOffB1, H1, nullptr, st);
-  layer<true, false>(M, kMlpHid, kMlpHid, H1, w + kMlpOffW2, p + kMlpOffB2, H2, nullptr, st);
-  layer<false, true>(M, kMlpHid, kMlpOut, H2, w + kMlpOffW3, p + kMlpOffB3, Y, X, st);
-}
-
-template <bool RELU, bool SKIP>
 void layer_bf16(int M, int N, const float* X, const uint16_t* W, const float* b, float* Y, const float* X0,
                 hipStream_t st) {
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
@@ -451,39 +485,31 @@ void forward_infer(int M, const float* X, float* H1, float* H2, float* Y, hipStr
   layer_bf16<false, true>(M, kMlpOut, H2, w + kMlpOffW3, p + kMlpOffB3, Y, X, st);
 }
 
-// g <- gradient of the batch loss; dY must already hold dL/dY; dH2, dH1 work
-void backward(int M, const float* X, const float* H1, const float* H2, const float* dY, float* dH2, float* dH1,
-              float* g, hipStream_t st) {
-  const float* wr = g_model.wr;
-  gemm_launch(colmajor<float>('N', 'T', kMlpHid, kMlpOut, M, 1.f, H2, kMlpHid, dY, kMlpOut, 0.f, g + kMlpOffW3,
-                              kMlpHid), st);
-  hipLaunchKernelGGL(rowsum_kernel, dim3(1), dim3(256), 0, st, kMlpOut, M, dY, g + kMlpOffB3);
-  gemm_launch(colmajor<float>('N', 'N', kMlpHid, M, kMlpOut, 1.f, wr + kMlpOffW3, kMlpHid, dY, kMlpOut, 0.f, dH2,
-                              kMlpHid), st);
-  hipLaunchKernelGGL(relu_mask_kernel, dim3(grid_of((int64_t)kMlpHid * M)), dim3(256), 0, st, (int64_t)kMlpHid * M, H2,
-                     dH2);
-  gemm_launch(colmajor<float>('N', 'T', kMlpHid, kMlpHid, M, 1.f, H1, kMlpHid, dH2, kMlpHid, 0.f, g + kMlpOffW2,
-                              kMlpHid), st);
-  hipLaunchKernelGGL(rowsum_kernel, dim3(1), dim3(256), 0, st, kMlpHid, M, dH2, g + kMlpOffB2);
-  gemm_launch(colmajor<float>('N', 'N', kMlpHid, M, kMlpHid, 1.f, wr + kMlpOffW2, kMlpHid, dH2, kMlpHid, 0.f, dH1,
-                              kMlpHid), st);
-  hipLaunchKernelGGL(relu_mask_kernel, dim3(grid_of((int64_t)kMlpHid * M)), dim3(256), 0, st, (int64_t)kMlpHid * M, H1,
-                     dH1);
-  gemm_launch(colmajor<float>('N', 'T', kMlpIn, kMlpHid, M, 1.f, X, kMlpIn, dH1, kMlpHid, 0.f, g + kMlpOffW1, kMlpIn),
-              st);
-  hipLaunchKernelGGL(rowsum_kernel, dim3(1), dim3(256), 0, st, kMlpHid, M, dH1, g + kMlpOffB1);
-  TTF_HIP(hipGetLastError());
+// Columns per slice of the gradient sums: at most kGradSlices slices, at
+// least 128 columns each and whole multiples of 64.
+int grad_slice(int M) {
+  const int64_t per = std::max<int64_t>(128, ((int64_t)M + kGradSlices - 1) / kGradSlices);
+  return (int)((per + 63) / 64 * 64);
 }
 
-// Workspace for M columns: X | H1 | H2 | Y | dY | dH2 | dH1 | scale (floats)
+// Work-groups (and loss partials) of the output layer.
+int64_t loss_parts(int M) { return kMlpOut / 32 * (((int64_t)M + 31) / 32); }
+
+// Workspace for M columns: X | H1 | H2 | Y | dY | dH2 | dH1 | scale
+// (floats); training: the loss partials and the gradient slices before them.
 struct MlpWork {
-  float *X, *H1, *H2, *Y, *dY, *dH2, *dH1, *scale;
+  float *X, *H1, *H2, *Y, *dY, *dH2, *dH1, *scale, *slices;
+  double* lpart;
 };
 MlpWork work_for(int M, bool train) {
   const size_t per = (size_t)kMlpIn + 2 * kMlpHid + kMlpOut + (train ? (size_t)kMlpOut + 2 * kMlpHid : 0) + 1;
-  float* base = (float*)arena(kArenaMlp, sizeof(float) * per * (size_t)M + 256);
+  const size_t nl = train ? ((size_t)loss_parts(M) + 1) / 2 * 2 : 0;   // keeps what follows on 16 bytes
+  const size_t ns = train ? (size_t)kMlpParams * kGradSlices : 0;
+  char* base = (char*)arena(kArenaMlp, sizeof(double) * nl + sizeof(float) * (ns + per * (size_t)M) + 256);
   MlpWork w{};
-  w.X = base;
+  w.lpart = (double*)base;
+  w.slices = (float*)(base + sizeof(double) * nl);
+  w.X = w.slices + ns;
   w.H1 = w.X + (size_t)kMlpIn * M;
   w.H2 = w.H1 + (size_t)kMlpHid * M;
   w.Y = w.H2 + (size_t)kMlpHid * M;
@@ -519,15 +545,47 @@ void set_params_device(const float* host) {
   g_model.ready = true;
 }
 
-double batch_loss_grad(int M, const float* X, const float* T, MlpWork& w, float* g, double* part, double* out,
-                       hipStream_t st) {
-  forward(M, X, w.H1, w.H2, w.Y, st);
-  const int64_t cnt = (int64_t)kMlpOut * M;
-  const int ng = std::min(grid_of(cnt), 256);
-  hipLaunchKernelGGL(loss_grad_kernel, dim3(ng), dim3(256), 0, st, cnt, M, w.Y, T, w.dY, part);
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(64), 0, st, ng, part, 1.0 / (double)cnt, out);
-  backward(M, X, w.H1, w.H2, w.dY, w.dH2, w.dH1, g, st);
-  return 0.0;
+// Loss (device) and gradient g of the batch (X, T); X on a 16-byte boundary.
+void batch_loss_grad(int M, const float* X, const float* T, MlpWork& w, float* g, double* loss, hipStream_t st) {
+  const float* p = g_model.master;
+  const float* wr = g_model.wr;
+  const double count = (double)kMlpOut * M;
+  auto op = [&](int rows, int K, const float* A, int64_t sAi, int64_t sAk, const float* B, float* C) {
+    GemmOp<float> o{};
+    o.M = rows; o.N = M; o.K = K;
+    o.A = A; o.sAi = sAi; o.sAk = sAk;
+    o.B = B; o.sBk = 1; o.sBj = K;
+    o.C = C;
+    return o;
+  };
+  auto grid = [&](int rows) { return dim3((unsigned)((int64_t)(rows / 32) * (((int64_t)M + 31) / 32))); };
+  const dim3 blk(256);
+  const float* no = nullptr;
+  double* nop = nullptr;
+  // forward: H = relu(W^T In + b), and the output layer with the loss
+  hipLaunchKernelGGL(train_layer_kernel<0>, grid(kMlpHid), blk, 0, st,
+                     op(kMlpHid, kMlpIn, wr + kMlpOffW1, kMlpIn, 1, X, w.H1), p + kMlpOffB1, no, no, 0.f, nop);
+  hipLaunchKernelGGL(train_layer_kernel<0>, grid(kMlpHid), blk, 0, st,
+                     op(kMlpHid, kMlpHid, wr + kMlpOffW2, kMlpHid, 1, w.H1, w.H2), p + kMlpOffB2, no, no, 0.f, nop);
+  hipLaunchKernelGGL(train_layer_kernel<1>, grid(kMlpOut), blk, 0, st,
+                     op(kMlpOut, kMlpHid, wr + kMlpOffW3, kMlpHid, 1, w.H2, w.dY), p + kMlpOffB3, X, T,
+                     2.0f / ((float)M * (float)kMlpOut), w.lpart);
+  // backward: dH = (W D) masked
+  hipLaunchKernelGGL(train_back_kernel, grid(kMlpHid), blk, 0, st,
+                     op(kMlpHid, kMlpOut, wr + kMlpOffW3, 1, kMlpHid, w.dY, w.dH2), (const float*)w.H2);
+  hipLaunchKernelGGL(train_back_kernel, grid(kMlpHid), blk, 0, st,
+                     op(kMlpHid, kMlpHid, wr + kMlpOffW2, 1, kMlpHid, w.dH2, w.dH1), (const float*)w.H1);
+  WeightGrads a{};
+  a.in[0] = X; a.in[1] = w.H1; a.in[2] = w.H2;
+  a.d[0] = w.dH1; a.d[1] = w.dH2; a.d[2] = w.dY;
+  a.M = M;
+  a.slice = grad_slice(M);
+  a.nslices = (int)(((int64_t)M + a.slice - 1) / a.slice);
+  hipLaunchKernelGGL(weight_grad_kernel, dim3((unsigned)(a.nslices * (kGradTiles + kGradRows))), blk, 0, st, a,
+                     w.slices);
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)((kMlpParams + 255) / 256 + 1)), blk, 0, st, a.nslices,
+                     (const float*)w.slices, g, (int)loss_parts(M), (const double*)w.lpart, 1.0 / count, loss);
+  TTF_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -630,10 +688,13 @@ int ttf_mlp_loss_grad(int M, const float* X, const float* T, double* loss, float
     TTF_REQUIRE(M > 0, "ttf_mlp_loss_grad: M=%d", M);
     hipStream_t st = stream();
     MlpWork w = work_for(M, true);
-    float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * 512);
-    double* part = (double*)(g + kMlpParams + (kMlpParams & 1));
-    double* out = part + 256;
-    batch_loss_grad(M, X, T, w, g, part, out, st);
+    float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * 2);
+    double* out = (double*)(g + kMlpParams + (kMlpParams & 1));
+    if ((reinterpret_cast<uintptr_t>(X) & 15) != 0) {
+      TTF_HIP(hipMemcpyAsync(w.X, X, sizeof(float) * (size_t)kMlpIn * M, hipMemcpyDeviceToDevice, st));
+      X = w.X;
+    }
+    batch_loss_grad(M, X, T, w, g, out, st);
     TTF_HIP(hipMemcpyAsync(loss, out, sizeof(double), hipMemcpyDeviceToHost, st));
     if (grad) read_back(grad, g, sizeof(float) * (size_t)kMlpParams, st);
   });
@@ -649,10 +710,9 @@ int ttf_mlp_train(long nsamples, const float* X, const float* T, int epochs, int
     const int B = (int)std::min<long>(batch, nsamples);
     const long nbat = nsamples / B;
     MlpWork w = work_for(B, true);
-    float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * (512 + nbat + 1) +
+    float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * (nbat + 1) +
                                              sizeof(int) * (size_t)nsamples + 64);
-    double* part = (double*)(g + kMlpParams + (kMlpParams & 1));
-    double* losses = part + 256;
+    double* losses = (double*)(g + kMlpParams + (kMlpParams & 1));
     int* idx = (int*)(losses + nbat + 1);
     float* Tb = (float*)arena(kArenaMlp3, sizeof(float) * (size_t)kMlpOut * B);   // batch targets
     std::vector<int> perm((size_t)nsamples);
@@ -669,7 +729,7 @@ int ttf_mlp_train(long nsamples, const float* X, const float* T, int epochs, int
         hipLaunchKernelGGL(gather_cols_kernel, dim3(grid_of((int64_t)kMlpIn * B)), dim3(256), 0, st, kMlpIn, B, ib, X, w.X);
         hipLaunchKernelGGL(gather_cols_kernel, dim3(grid_of((int64_t)kMlpOut * B)), dim3(256), 0, st, kMlpOut, B, ib, T,
                            Tb);
-        batch_loss_grad(B, w.X, Tb, w, g, part, losses + bi, st);
+        batch_loss_grad(B, w.X, Tb, w, g, losses + bi, st);
         ++g_model.step;
         const float c1 = 1.f - std::pow(beta1, (float)g_model.step);
         const float c2 = 1.f - std::pow(beta2, (float)g_model.step);
