@@ -48,32 +48,21 @@ __global__ void axpby_kernel(int64_t n, double a, const double* __restrict__ x, 
 // (tt_linalg.f90:397-491).  d1(b1, a1) = Phi1(b1, b1, a1), d2(b2, a2) =
 // Phi2(b2, a2, b2); A(a1, i, j, a2).
 //  'c': block (b1, b2) of size n: M(i, j) = sum d1(b1,a1) A(a1,i,j,a2) d2(b2,a2),
-//       stored at (b2 + rx2 b1) n^2 (layout (n, n, rx2, rx1));
+//       stored at (b2 + rx2 b1) n^2 (layout (n, n, rx2, rx1)), formed as a product (jac_gen);
 //  'l': block b2 of size rx1 n: M((c1,i),(b1,j)) = sum Phi1(c1,b1,a1) A d2(b2,a2);
 //  'r': block b1 of size n rx2: M((i,c2),(j,b2)) = sum d1(b1,a1) A Phi2(b2,a2,c2).
 __global__ void jac_blocks_kernel(char type, int rx1, int n, int rx2, int ra1, int ra2,
                                   const double* __restrict__ Phi1, const double* __restrict__ A,
                                   const double* __restrict__ Phi2, double* __restrict__ M) {
   int64_t bs, nblk;
-  if (type == 'c') { bs = n; nblk = (int64_t)rx1 * rx2; }
-  else if (type == 'l') { bs = (int64_t)rx1 * n; nblk = rx2; }
+  if (type == 'l') { bs = (int64_t)rx1 * n; nblk = rx2; }
   else { bs = (int64_t)n * rx2; nblk = rx1; }
   const int64_t total = bs * bs * nblk;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t row = e % bs, col = (e / bs) % bs, blk = e / (bs * bs);
     double s = 0.0;
-    if (type == 'c') {
-      const int i = (int)row, j = (int)col, b2 = (int)(blk % rx2), b1 = (int)(blk / rx2);
-      for (int a2 = 0; a2 < ra2; ++a2) {
-        const double d2 = Phi2[b2 + (int64_t)rx2 * (a2 + (int64_t)ra2 * b2)];
-        double t = 0.0;
-        for (int a1 = 0; a1 < ra1; ++a1)
-          t += Phi1[b1 + (int64_t)rx1 * (b1 + (int64_t)rx1 * a1)] *
-               A[a1 + (int64_t)ra1 * (i + (int64_t)n * (j + (int64_t)n * a2))];
-        s += t * d2;
-      }
-    } else if (type == 'l') {
+    if (type == 'l') {
       const int c1 = (int)(row % rx1), i = (int)(row / rx1), b1 = (int)(col % rx1), j = (int)(col / rx1);
       const int b2 = (int)blk;
       for (int a2 = 0; a2 < ra2; ++a2) {
@@ -97,6 +86,28 @@ __global__ void jac_blocks_kernel(char type, int rx1, int n, int rx2, int ra1, i
       }
     }
     M[e] = s;
+  }
+}
+
+// The two operands of the 'c' blocks as one product over the bond indices,
+//   M((i,j), b) = sum_{a1,a2} P((i,j), a1 + ra1 a2) D(a1 + ra1 a2, b),
+// b = b2 + rx2 b1: P is A with its bond indices last, D(., b) = d1(b1, a1)
+// d2(b2, a2).  One thread per entry of P, then of D.
+__global__ __launch_bounds__(256) void jac_c_operands_kernel(int rx1, int n, int rx2, int ra1, int ra2,
+                                                             const double* __restrict__ Phi1,
+                                                             const double* __restrict__ A,
+                                                             const double* __restrict__ Phi2,
+                                                             double* __restrict__ P, double* __restrict__ D) {
+  const int64_t nn = (int64_t)n * n, np = nn * ra1 * ra2, nk = (int64_t)ra1 * ra2;
+  const int64_t total = np + nk * rx1 * rx2;
+  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
+    if (e < np) {
+      const int64_t ij = e % nn, k = e / nn, a1 = k % ra1, a2 = k / ra1;
+      P[e] = A[a1 + ra1 * (ij + nn * a2)];
+    } else {
+      const int64_t f = e - np, k = f % nk, b = f / nk, a1 = k % ra1, a2 = k / ra1, b2 = b % rx2, b1 = b / rx2;
+      D[f] = Phi1[b1 + rx1 * (b1 + rx1 * a1)] * Phi2[b2 + rx2 * (a2 + ra2 * b2)];
+    }
   }
 }
 
@@ -181,63 +192,90 @@ __global__ __launch_bounds__(256) void batched_inverse_kernel(int n, double* __r
   for (int e = tid; e < n * n; e += nt) g[(e % n) + ldm * (e / n)] = a[(e % n) + ld * (e / n)];
 }
 
-// In-place inverse of symmetric positive definite n x n blocks (n <= 128;
+// In-place inverse of symmetric positive definite n x n blocks (n <= 16 TS;
 // block b at M + b stride, leading dimension ldm) by Gauss-Jordan
 // elimination without pivoting, one work-group of 256 per block with the
-// block in registers: thread t owns the 8 x 8 tile at rows 8 (t % 16) and
-// columns 8 (t / 16) of the block padded to order 128 with the identity.
+// block in registers: thread t owns the TS x TS tile at rows TS (t % 16) and
+// columns TS (t / 16) of the block padded to order 16 TS with the identity.
 // Step k broadcasts column k and row k through LDS, double-buffered so that
 // each step has one barrier.  The pivots are those of the LDL^T
 // factorisation, all positive exactly when the block is positive definite;
 // a pivot that is not positive sets info[b] and leaves the block as it
-// was.  A block whose info[b] is already set is skipped.
+// was.  A block whose info[b] is already set is skipped.  With CHECK a block
+// that is not exactly symmetric is treated like one that is not positive
+// definite.
+//
+// The work per step is the padded block's, so the tile follows the order:
+// 4096 blocks of order 64 took 489 us in tiles of 8 x 8 (padded to 128) and
+// 47 us for a symmetry check of its own, and take 173 us in tiles of 4 x 4
+// with the check (the blocks' 268 MB in and out alone are 52 us).
+template <int TS, bool CHECK>
 __global__ __launch_bounds__(256) void spd_inverse_tiled_kernel(int n, double* __restrict__ M, int64_t ldm,
                                                                 int64_t stride, int* __restrict__ info) {
-  __shared__ double colb[2][128];
-  __shared__ double rowb[2][128];
+  __shared__ double colb[2][16 * TS];
+  __shared__ double rowb[2][16 * TS];
   if (info[blockIdx.x] != 0) return;   // uniform
   const int t = threadIdx.x, ti = t & 15, tj = t >> 4;
   double* g = M + (int64_t)blockIdx.x * stride;
-  double a[8][8];
+  double a[TS][TS];
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
+  for (int s = 0; s < TS; ++s)
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int i = 8 * ti + r, j = 8 * tj + s;
-      a[r][s] = (i < n && j < n) ? g[i + ldm * j] : (i == j ? 1.0 : 0.0);
+    for (int r = 0; r < TS; ++r) {
+      // entries past the block read a clamped one (a load under its own
+      // condition becomes a branch with a full wait)
+      const int i = TS * ti + r, j = TS * tj + s;
+      const double v = g[min(i, n - 1) + ldm * min(j, n - 1)];
+      a[r][s] = (i < n && j < n) ? v : (i == j ? 1.0 : 0.0);
     }
   bool bad = false;
-  const int nkb = (n + 7) / 8;
+  if constexpr (CHECK) {
+    bool differ = false;
+#pragma unroll
+    for (int s = 0; s < TS; ++s)
+#pragma unroll
+      for (int r = 0; r < TS; ++r) {
+        const int i = TS * ti + r, j = TS * tj + s;
+        const double v = g[min(j, n - 1) + ldm * min(i, n - 1)];
+        differ = differ || (i < n && j < n && a[r][s] != v);
+      }
+    bad = __syncthreads_or(differ ? 1 : 0) != 0;
+    if (bad) {   // uniform
+      if (t == 0) info[blockIdx.x] = 1;
+      return;
+    }
+  }
+  const int nkb = (n + TS - 1) / TS;
   for (int kb = 0; kb < nkb; ++kb) {
     const bool rowk = ti == kb, colk = tj == kb;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int k = 8 * kb + c;
+    for (int c = 0; c < TS; ++c) {
+      const int k = TS * kb + c;
       if (k < n) {   // uniform
         const int buf = k & 1;
         if (colk) {
 #pragma unroll
-          for (int r = 0; r < 8; ++r) colb[buf][8 * ti + r] = a[r][c];
+          for (int r = 0; r < TS; ++r) colb[buf][TS * ti + r] = a[r][c];
         }
         if (rowk) {
 #pragma unroll
-          for (int s = 0; s < 8; ++s) rowb[buf][8 * tj + s] = a[c][s];
+          for (int s = 0; s < TS; ++s) rowb[buf][TS * tj + s] = a[c][s];
         }
         __syncthreads();
         const double pv = rowb[buf][k];
         bad = bad || !(pv > 0.0);
         const double inv = 1.0 / pv;
-        double f[8], h[8];
+        double f[TS], h[TS];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) f[r] = colb[buf][8 * ti + r];
+        for (int r = 0; r < TS; ++r) f[r] = colb[buf][TS * ti + r];
 #pragma unroll
-        for (int s = 0; s < 8; ++s) h[s] = rowb[buf][8 * tj + s] * inv;
+        for (int s = 0; s < TS; ++s) h[s] = rowb[buf][TS * tj + s] * inv;
         // a(i, j) - a(i, k) a(k, j) / pv off row and column k; row k scaled
         // by 1 / pv; column k -a(i, k) / pv; the pivot 1 / pv
 #pragma unroll
-        for (int r = 0; r < 8; ++r)
+        for (int r = 0; r < TS; ++r)
 #pragma unroll
-          for (int s = 0; s < 8; ++s) {
+          for (int s = 0; s < TS; ++s) {
             double v = a[r][s] - f[r] * h[s];
             if (s == c && colk) v = -f[r] * inv;
             if (r == c && rowk) v = (s == c && colk) ? inv : h[s];
@@ -252,25 +290,22 @@ __global__ __launch_bounds__(256) void spd_inverse_tiled_kernel(int n, double* _
     return;
   }
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
+  for (int s = 0; s < TS; ++s)
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int i = 8 * ti + r, j = 8 * tj + s;
+    for (int r = 0; r < TS; ++r) {
+      const int i = TS * ti + r, j = TS * tj + s;
       if (i < n && j < n) g[i + ldm * j] = a[r][s];
     }
 }
 
-// flag[b] = 1 unless block b (n x n, consecutive blocks of n^2) is exactly
-// symmetric with a positive diagonal; one work-group per block.
-__global__ __launch_bounds__(256) void sym_check_kernel(int n, const double* __restrict__ M, int* __restrict__ flag) {
-  const double* g = M + (int64_t)blockIdx.x * n * n;
-  bool bad = false;
-  for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-    const int i = e % n, j = e / n;
-    if (i < j) bad = bad || g[i + (int64_t)n * j] != g[j + (int64_t)n * i];
-    else if (i == j) bad = bad || !(g[i + (int64_t)n * i] > 0.0);
-  }
-  if (bad) flag[blockIdx.x] = 1;   // every writer stores the same value
+// The smallest tile whose 16 x 16 grid covers the order.
+template <bool CHECK>
+void spd_inverse_launch(int n, double* M, int64_t ldm, int64_t stride, int64_t nblk, int* info, hipStream_t st) {
+  const dim3 grid((unsigned)nblk), blk(256);
+  if (n <= 32) hipLaunchKernelGGL((spd_inverse_tiled_kernel<2, CHECK>), grid, blk, 0, st, n, M, ldm, stride, info);
+  else if (n <= 64) hipLaunchKernelGGL((spd_inverse_tiled_kernel<4, CHECK>), grid, blk, 0, st, n, M, ldm, stride, info);
+  else hipLaunchKernelGGL((spd_inverse_tiled_kernel<8, CHECK>), grid, blk, 0, st, n, M, ldm, stride, info);
+  TTF_HIP(hipGetLastError());
 }
 
 // y(blk) = J(blk) x(blk) for all blocks: block b has size bs, matrix at
@@ -327,9 +362,29 @@ void jac_gen(char type, int rx1, int n, int rx2, int ra1, int ra2, const double*
   TTF_REQUIRE(bs <= kInvMaxN, "djac_gen: block size %d exceeds %d for ptype '%c'", bs, kInvMaxN, type);
   TTF_REQUIRE(nblk <= 0x7fffffff, "djac_gen: too many blocks");
   const int64_t total = (int64_t)bs * bs * nblk;
-  hipLaunchKernelGGL(jac_blocks_kernel, dim3(grid_for(total)), dim3(256), 0, st, type, rx1, n, rx2, ra1, ra2,
-                     Phi1, A, Phi2, jacs);
-  TTF_HIP(hipGetLastError());
+  if (type == 'c') {
+    // every entry is a sum over the ra1 ra2 bond pairs, so the blocks are a
+    // product of n^2 x (ra1 ra2) by (ra1 ra2) x (rx1 rx2) on the matrix
+    // cores, bound by writing the blocks: 4096 blocks of order 64 with 36
+    // bond pairs take 46 us, where one thread per entry took 696.  Entries
+    // (i, j) and (j, i) are the same sums in the same order, so the blocks
+    // of a symmetric operator stay exactly symmetric.
+    const int64_t nk = (int64_t)ra1 * ra2, nn = (int64_t)n * n;
+    double* P = (double*)arena(kArenaSolver2, sizeof(double) * (size_t)(nk * (nn + nblk)));
+    double* D = P + nk * nn;
+    hipLaunchKernelGGL(jac_c_operands_kernel, dim3(grid_for(nk * (nn + nblk))), dim3(256), 0, st, rx1, n, rx2, ra1,
+                       ra2, Phi1, A, Phi2, P, D);
+    TTF_HIP(hipGetLastError());
+    // the ranks change from one local problem to the next: no tuning runs
+    // for products that may be formed once
+    GemmOp<double> g = colmajor<double>('N', 'N', (int)nn, (int)nblk, (int)nk, 1.0, P, nn, D, nk, 0.0, jacs, nn);
+    const size_t ws = gemm_workspace(g);
+    gemm_launch_ws(g, ws ? (double*)arena(kArenaSplitK, sizeof(double) * ws) : nullptr, ws, st);
+  } else {
+    hipLaunchKernelGGL(jac_blocks_kernel, dim3(grid_for(total)), dim3(256), 0, st, type, rx1, n, rx2, ra1, ra2,
+                       Phi1, A, Phi2, jacs);
+    TTF_HIP(hipGetLastError());
+  }
   int* info = (int*)arena(kArenaSmall, sizeof(int) * (size_t)nblk * 2);
   int* other = info + nblk;   // blocks left to the pivoting kernel
   TTF_HIP(hipMemsetAsync(info, 0, sizeof(int) * (size_t)nblk * 2, st));
@@ -346,9 +401,7 @@ void jac_gen(char type, int rx1, int n, int rx2, int ra1, int ra2, const double*
   // pivoting; the others, and any that turns out not positive definite,
   // through Gauss-Jordan with partial pivoting.  Both are the inverse to
   // rounding, which is all dgesv's solve promises.
-  hipLaunchKernelGGL(sym_check_kernel, dim3((unsigned)nblk), dim3(256), 0, st, bs, jacs, other);
-  hipLaunchKernelGGL(spd_inverse_tiled_kernel, dim3((unsigned)nblk), dim3(256), 0, st, bs, jacs, (int64_t)bs,
-                     (int64_t)bs * bs, other);
+  spd_inverse_launch<true>(bs, jacs, bs, (int64_t)bs * bs, nblk, other, st);
   hipLaunchKernelGGL(batched_inverse_kernel, dim3((unsigned)nblk), dim3(256), lds, st, bs, jacs, (int64_t)bs,
                      (int64_t)bs * bs, info, (const int*)other);
   TTF_HIP(hipGetLastError());
@@ -401,9 +454,7 @@ bool spd_block_inverse(int nb, int64_t nblk, double* M, hipStream_t st) {
   int* info = (int*)(ws + sizeof(double) * (size_t)(hh * nblk));
   TTF_HIP(hipMemsetAsync(info, 0, sizeof(int) * (size_t)nblk, st));
   auto inv = [&](int n, double* base) {
-    hipLaunchKernelGGL(spd_inverse_tiled_kernel, dim3((unsigned)nblk), dim3(256), 0, st, n, base, (int64_t)nb, nb2,
-                       info);
-    TTF_HIP(hipGetLastError());
+    spd_inverse_launch<false>(n, base, nb, nb2, nblk, info, st);
   };
   auto batched = [&](GemmOp<double> g, int64_t sa, int64_t sb, int64_t sc) {
     g.nb0 = (int)nblk;
