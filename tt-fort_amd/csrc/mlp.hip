@@ -300,119 +300,219 @@ __global__ __launch_bounds__(256) void grad_reduce_kernel(int nslices, const flo
   g[e] = sum;
 }
 
-// The inference form of the layers on gfx950's bf16 matrix cores: the same
-// Y = act(W^T X + b) (+ the point-Jacobi term with SKIP), with the
-// activations X rounded to bf16 (round to nearest even) and the products
-// accumulated in fp32 by v_mfma_f32_16x16x32_bf16.  K = 256 for every layer
-// of the network.  Lane l feeds row (or column) l % 16 and the eight
-// consecutive k = 8 (l / 16) .. +7 of each 32-deep step to both operands,
-// so the A and B elements it supplies meet at the same k; fragments are
-// read straight from global memory (weights 16 bytes, activations 32 bytes
-// per lane), all eight k-steps' loads issued before the products.
+// ---- inference: the whole network in one launch on gfx950's bf16 matrix
+// cores, with the activations rounded to bf16 (round to nearest even) at
+// each layer's input and the products accumulated in fp32 by
+// v_mfma_f32_16x16x32_bf16.  Lane l feeds row (or column) l % 16 and the
+// eight consecutive k = 8 (l / 16) .. +7 of each 32-deep step to both
+// operands, so the A and B elements it supplies meet at the same k.
+//
+// A work-group of eight waves takes 16 columns through all three layers,
+// the activations in LDS and the weights (288 KB in bf16) from L2: 16
+// columns make 256 work-groups of the 4096 blocks of a rank 64 x 64 problem.
+// What bounds it is latency, so each layer's weights are requested a phase
+// before they are used.  Separate feature, layer and scatter kernels took 43
+// + 32 + 5 us for those blocks (the features' strided reads of A's diagonals
+// most of it); with the diagonals packed first and everything in one kernel
+// the apply takes 22 us instead of 78.
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf4_t __attribute__((ext_vector_type(4)));
 constexpr int kBfK = 256;
-static_assert(kMlpIn == kBfK && kMlpHid == kBfK, "the bf16 layers assume K = 256");
+static_assert(kMlpIn == kBfK && kMlpHid == kBfK && kMlpOut == 64, "the inference kernel's layer sizes");
+constexpr int kInfCols = 16, kInfWaves = 8, kInfThreads = 64 * kInfWaves;
+constexpr int kActLd = kBfK + 8;   // bf16 per column of activations: 16-byte rows, spread over the banks
 
-template <bool RELU, bool SKIP>
-__global__ __launch_bounds__(256) void layer_bf16_kernel(int M, int N, const float* __restrict__ X,
-                                                         const uint16_t* __restrict__ W,
-                                                         const float* __restrict__ bias, float* __restrict__ Y,
-                                                         const float* __restrict__ X0) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wn = wave & 1, wm = wave >> 1;
-  const int n0 = blockIdx.x * 64 + wn * 32, m0 = blockIdx.y * 64 + wm * 32;
-  const int g = lane >> 4, c = lane & 15;
-  f4_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-  const uint16_t* wa[2];
-  const float* xb[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int n = min(n0 + 16 * i + c, N - 1);   // rows past N are computed and not stored
-    wa[i] = W + 8 * g + (int64_t)kBfK * n;
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int m = min(m0 + 16 * j + c, M - 1);
-    xb[j] = X + 8 * g + (int64_t)kBfK * m;
-  }
-  uint4 wr[kBfK / 32][2];
-  float4 xr[kBfK / 32][2][2];
-#pragma unroll
-  for (int s = 0; s < kBfK / 32; ++s) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) wr[s][i] = *reinterpret_cast<const uint4*>(wa[i] + 32 * s);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      xr[s][j][0] = *reinterpret_cast<const float4*>(xb[j] + 32 * s);
-      xr[s][j][1] = *reinterpret_cast<const float4*>(xb[j] + 32 * s + 4);
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < kBfK / 32; ++s) {
-    bf8_t a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = __builtin_bit_cast(bf8_t, wr[s][i]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float4 lo = xr[s][j][0], hi = xr[s][j][1];
-      b[j] = bf8_t{(__bf16)lo.x, (__bf16)lo.y, (__bf16)lo.z, (__bf16)lo.w,
-                   (__bf16)hi.x, (__bf16)hi.y, (__bf16)hi.z, (__bf16)hi.w};
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-  }
-  // the epilogue's operands for the 16 outputs (bias, and with SKIP the
-  // block diagonal and the residual), loaded from clamped in-range indices
-  // before any is used: loaded under each output's own condition they
-  // become a branch with a full wait apiece
-  float eb[16], ed[16], ex[16];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int q = i * 8 + j * 4 + r;
-        const int gn = min(n0 + i * 16 + mfma_row<float>(lane, r), N - 1);
-        const int gm = min(m0 + j * 16 + c, M - 1);
-        eb[q] = bias[gn];
-        if (SKIP) {
-          ed[q] = X0[gn + (int64_t)kMlpIn * gm];
-          ex[q] = X0[3 * kMlpBlock + gn + (int64_t)kMlpIn * gm];
-        }
-      }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int q = i * 8 + j * 4 + r;
-        const int gn = n0 + i * 16 + mfma_row<float>(lane, r);
-        const int gm = m0 + j * 16 + c;
-        if (gn < N && gm < M) {
-          float val = acc[i][j][r] + eb[q];
-          if (RELU) val = fmaxf(val, 0.f);
-          if (SKIP) val += ed[q] != 0.f ? ex[q] / ed[q] : 0.f;
-          Y[gn + (int64_t)N * gm] = val;
-        }
-      }
+// The three central diagonals of A's bond slices: Ad[k][q][i], k = a1 ra2 +
+// a2, q = diagonal, super-, subdiagonal (zero past the edge).
+__global__ __launch_bounds__(192) void diagonals_kernel(int n, int ra1, int ra2, const double* __restrict__ A,
+                                                        double* __restrict__ Ad) {
+  const int a1 = blockIdx.x / ra2, a2 = blockIdx.x - a1 * ra2;
+  const int q = threadIdx.x >> 6, i = threadIdx.x & 63;
+  const int row = q == 2 ? i + 1 : i, col = q == 1 ? i + 1 : i;
+  const bool in = row < n && col < n;
+  const double v = A[a1 + ra1 * (min(row, n - 1) + (int64_t)n * (min(col, n - 1) + (int64_t)n * a2))];
+  Ad[192 * (int64_t)blockIdx.x + threadIdx.x] = in ? v : 0.0;
 }
 
-// z(b1, i, b2) = Y(i, b) * scale(b), one wave per block
-__global__ __launch_bounds__(256) void scatter_kernel(int rx1, int n, int rx2, const float* __restrict__ Y,
-                                                      const float* __restrict__ scale, double* __restrict__ z) {
-  const int lane = threadIdx.x & 63;
-  const int64_t b = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-  if (b >= (int64_t)rx1 * rx2) return;
-  const int b1 = (int)(b % rx1), b2 = (int)(b / rx1);
-  z[b1 + (int64_t)rx1 * (lane + (int64_t)n * b2)] = (double)Y[lane + (int64_t)kMlpOut * b] * (double)scale[b];
+struct InferArgs {
+  int ncols;
+  const uint16_t* w;     // bf16 parameters
+  const float* master;   // fp32 parameters (biases)
+  // columns from X (kMlpIn x ncols) to Y (kMlpOut x ncols)
+  const float* X;
+  float* Y;
+  // or the blocks of the local vector v (rx1, 64, rx2), corrections to z
+  int rx1, rx2, ra1, ra2;
+  const double* phi1;
+  const double* Ad;
+  const double* phi2;
+  const double* v;
+  double* z;
+};
+
+// One 16-row group of W^T act(:, 16 columns): fragments from registers (w)
+// and LDS.
+__device__ __forceinline__ f4_t infer_rows(const uint4 (&w)[kBfK / 32], const __bf16* act) {
+  f4_t acc = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kBfK / 32; ++s)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, w[s]),
+                                                  *reinterpret_cast<const bf8_t*>(act + 32 * s), acc, 0, 0, 0);
+  return acc;
+}
+
+template <bool BLOCKS>
+__global__ __launch_bounds__(kInfThreads, 2) void infer_kernel(InferArgs a) {
+  __shared__ __attribute__((aligned(16))) __bf16 act[2][kInfCols * kActLd];
+  __shared__ float skip_d[kInfCols][kMlpBlock + 1], skip_r[kInfCols][kMlpBlock + 1];
+  __shared__ float scale[kInfCols];
+  __shared__ double rs[BLOCKS ? kInfCols : 1][kMlpBlock + 1];
+  __shared__ double cs[BLOCKS ? kInfCols : 1][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int col0 = blockIdx.x * kInfCols;
+  // wave w owns rows 32 w .. 32 w + 31 of the hidden layers
+  auto weights = [&](int64_t off, int row, uint4 (&w)[kBfK / 32]) {
+    const uint16_t* p = a.w + off + 8 * g + (int64_t)kBfK * (row + c);
+#pragma unroll
+    for (int s = 0; s < kBfK / 32; ++s) w[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
+  };
+  uint4 w1[2][kBfK / 32];
+  weights(kMlpOffW1, 32 * wave, w1[0]);
+  weights(kMlpOffW1, 32 * wave + 16, w1[1]);
+
+  if constexpr (BLOCKS) {
+    // residual slices: consecutive columns are consecutive in memory
+    const int64_t nblk = (int64_t)a.rx1 * a.rx2;
+    for (int e = tid; e < kInfCols * kMlpBlock; e += kInfThreads) {
+      const int cc = e & (kInfCols - 1), i = e / kInfCols;
+      const int64_t b = min((int64_t)col0 + cc, nblk - 1);
+      const int64_t b2 = b / a.rx1, b1 = b - b2 * a.rx1;
+      rs[cc][i] = a.v[b1 + a.rx1 * (i + (int64_t)kMlpBlock * b2)];
+    }
+    // the blocks' diagonals: this wave's two columns, bond pairs in the order
+    // of k, 64 coefficients at a time through LDS
+    const int nk = a.ra1 * a.ra2, q0 = 2 * wave;
+    double dg[2] = {0.0, 0.0}, up[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
+    for (int k0 = 0; k0 < nk; k0 += 64) {
+      const int k = min(k0 + lane, nk - 1), a1 = k / a.ra2, a2 = k - a1 * a.ra2;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int64_t b = min((int64_t)col0 + q0 + u, nblk - 1);
+        const int64_t b2 = b / a.rx1, b1 = b - b2 * a.rx1;
+        cs[q0 + u][lane] = a.phi1[b1 + a.rx1 * (b1 + a.rx1 * (int64_t)a1)] *
+                           a.phi2[b2 + a.rx2 * (a2 + a.ra2 * b2)];
+      }
+      __syncthreads();
+      const double* ad = a.Ad + 192 * (int64_t)k0 + lane;
+      const int kn = min(64, nk - k0);
+      for (int k4 = 0; k4 < kn; k4 += 4) {   // four bond pairs' loads in flight
+        double d[4][3];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) d[t][q] = ad[192 * min(k4 + t, kn - 1) + 64 * q];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          if (k4 + t < kn) {   // uniform
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const double cc = cs[q0 + u][k4 + t];
+              dg[u] += cc * d[t][0];
+              up[u] += cc * d[t][1];
+              lo[u] += cc * d[t][2];
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int q = q0 + u;
+      const double r = rs[q][lane];
+      const double sm = wave_sum(fabs(dg[u])) / kMlpBlock;
+      const double rn = sqrt(wave_sum(r * r));
+      const double sinv = sm > 0.0 ? 1.0 / sm : 0.0;
+      const double rinv = rn > 0.0 ? 1.0 / rn : 0.0;
+      const float fd = (float)(dg[u] * sinv), fr = (float)(r * rinv);
+      __bf16* x = act[0] + q * kActLd + lane;
+      x[0] = (__bf16)fd;
+      x[kMlpBlock] = (__bf16)(float)(up[u] * sinv);
+      x[2 * kMlpBlock] = (__bf16)(float)(lo[u] * sinv);
+      x[3 * kMlpBlock] = (__bf16)fr;
+      skip_d[q][lane] = fd;
+      skip_r[q][lane] = fr;
+      if (lane == 0) scale[q] = (float)(rn * sinv);
+    }
+  } else {
+    // two columns per wave, four features per lane
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int q = 2 * wave + u;
+      const float* x = a.X + (int64_t)kMlpIn * min(col0 + q, a.ncols - 1) + lane;
+      float f[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) f[t] = x[64 * t];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) act[0][q * kActLd + 64 * t + lane] = (__bf16)f[t];
+      skip_d[q][lane] = f[0];
+      skip_r[q][lane] = f[3];
+    }
+  }
+
+  // hidden layers: rows 32 wave + 16 i + 4 g + r, column c
+  auto hidden = [&](const uint4 (&w)[2][kBfK / 32], int64_t bias, const __bf16* in, __bf16* out) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = 32 * wave + 16 * i + 4 * g;
+      const float* pb = a.master + bias + row;
+      const float b[4] = {pb[0], pb[1], pb[2], pb[3]};
+      const f4_t acc = infer_rows(w[i], in + c * kActLd + 8 * g);
+      bf4_t h;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h[r] = (__bf16)fmaxf(acc[r] + b[r], 0.f);
+      *reinterpret_cast<bf4_t*>(out + c * kActLd + row) = h;
+    }
+  };
+  uint4 w2[2][kBfK / 32];
+  weights(kMlpOffW2, 32 * wave, w2[0]);
+  weights(kMlpOffW2, 32 * wave + 16, w2[1]);
+  __syncthreads();
+  hidden(w1, kMlpOffB1, act[0], act[1]);
+  uint4 w3[kBfK / 32];
+  weights(kMlpOffW3, 16 * (wave & 3), w3);
+  __syncthreads();
+  hidden(w2, kMlpOffB2, act[1], act[0]);
+  __syncthreads();
+  // output layer: waves 0..3, 16 rows each
+  float y[4];
+  const int row = 16 * (wave & 3) + 4 * g;
+  if (wave < 4) {   // uniform
+    const float* pb = a.master + kMlpOffB3 + row;
+    const f4_t acc = infer_rows(w3, act[0] + c * kActLd + 8 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float d = skip_d[c][row + r];
+      y[r] = acc[r] + pb[r];
+      y[r] += d != 0.f ? skip_r[c][row + r] / d : 0.f;
+    }
+  }
+  if constexpr (BLOCKS) {
+    const int64_t b = (int64_t)col0 + c;
+    if (wave < 4 && b < a.ncols) {
+      const int64_t b2 = b / a.rx1, b1 = b - b2 * a.rx1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        a.z[b1 + a.rx1 * (row + r + (int64_t)kMlpBlock * b2)] = (double)y[r] * (double)scale[c];
+    }
+  } else {
+    if (wave < 4 && col0 + c < a.ncols) {
+      float* dst = a.Y + (int64_t)kMlpOut * (col0 + c) + row;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[r] = y[r];
+    }
+  }
 }
 
 // T(i, c) = z(b1, i, b2) * inv(c) for the sampled blocks
@@ -466,25 +566,6 @@ void features(int rx1, int n, int rx2, int ra1, int ra2, const double* phi1, con
   TTF_HIP(hipGetLastError());
 }
 
-template <bool RELU, bool SKIP>
-void layer_bf16(int M, int N, const float* X, const uint16_t* W, const float* b, float* Y, const float* X0,
-                hipStream_t st) {
-  dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  hipLaunchKernelGGL((layer_bf16_kernel<RELU, SKIP>), grid, dim3(256), 0, st, M, N, X, W, b, Y, X0);
-  TTF_HIP(hipGetLastError());
-}
-
-// Inference: the same network with bf16 activations on the bf16 matrix
-// cores (training keeps the fp32 forward above, whose activations the
-// backward pass differentiates)
-void forward_infer(int M, const float* X, float* H1, float* H2, float* Y, hipStream_t st) {
-  const uint16_t* w = g_model.wbf;
-  const float* p = g_model.master;
-  layer_bf16<true, false>(M, kMlpHid, X, w + kMlpOffW1, p + kMlpOffB1, H1, nullptr, st);
-  layer_bf16<true, false>(M, kMlpHid, H1, w + kMlpOffW2, p + kMlpOffB2, H2, nullptr, st);
-  layer_bf16<false, true>(M, kMlpOut, H2, w + kMlpOffW3, p + kMlpOffB3, Y, X, st);
-}
-
 // Columns per slice of the gradient sums: at most kGradSlices slices, at
 // least 128 columns each and whole multiples of 64.
 int grad_slice(int M) {
@@ -495,32 +576,26 @@ int grad_slice(int M) {
 // Work-groups (and loss partials) of the output layer.
 int64_t loss_parts(int M) { return kMlpOut / 32 * (((int64_t)M + 31) / 32); }
 
-// Workspace for M columns: X | H1 | H2 | Y | dY | dH2 | dH1 | scale
-// (floats); training: the loss partials and the gradient slices before them.
+// Training workspace for M columns: the loss partials, the gradient slices
+// and (floats) X | H1 | H2 | dY | dH2 | dH1.
 struct MlpWork {
-  float *X, *H1, *H2, *Y, *dY, *dH2, *dH1, *scale, *slices;
+  float *X, *H1, *H2, *dY, *dH2, *dH1, *slices;
   double* lpart;
 };
-MlpWork work_for(int M, bool train) {
-  const size_t per = (size_t)kMlpIn + 2 * kMlpHid + kMlpOut + (train ? (size_t)kMlpOut + 2 * kMlpHid : 0) + 1;
-  const size_t nl = train ? ((size_t)loss_parts(M) + 1) / 2 * 2 : 0;   // keeps what follows on 16 bytes
-  const size_t ns = train ? (size_t)kMlpParams * kGradSlices : 0;
-  char* base = (char*)arena(kArenaMlp, sizeof(double) * nl + sizeof(float) * (ns + per * (size_t)M) + 256);
+MlpWork work_for(int M) {
+  const size_t per = (size_t)kMlpIn + 4 * kMlpHid + kMlpOut;
+  const size_t nl = ((size_t)loss_parts(M) + 1) / 2 * 2;   // keeps what follows on 16 bytes
+  const size_t ns = (size_t)kMlpParams * kGradSlices;
+  char* base = (char*)arena(kArenaMlp, sizeof(double) * nl + sizeof(float) * (ns + per * (size_t)M));
   MlpWork w{};
   w.lpart = (double*)base;
   w.slices = (float*)(base + sizeof(double) * nl);
   w.X = w.slices + ns;
   w.H1 = w.X + (size_t)kMlpIn * M;
   w.H2 = w.H1 + (size_t)kMlpHid * M;
-  w.Y = w.H2 + (size_t)kMlpHid * M;
-  float* p = w.Y + (size_t)kMlpOut * M;
-  if (train) {
-    w.dY = p;
-    w.dH2 = w.dY + (size_t)kMlpOut * M;
-    w.dH1 = w.dH2 + (size_t)kMlpHid * M;
-    p = w.dH1 + (size_t)kMlpHid * M;
-  }
-  w.scale = p;
+  w.dY = w.H2 + (size_t)kMlpHid * M;
+  w.dH2 = w.dY + (size_t)kMlpOut * M;
+  w.dH1 = w.dH2 + (size_t)kMlpHid * M;
   return w;
 }
 
@@ -599,10 +674,16 @@ void mlp_precond(int rx1, int n, int rx2, int ra1, int ra2, const double* phi1, 
   const int64_t nb64 = (int64_t)rx1 * rx2;
   TTF_REQUIRE(nb64 <= (1 << 24), "learned preconditioner: %lld blocks", (long long)nb64);
   const int nb = (int)nb64;
-  MlpWork w = work_for(nb, false);
-  features(rx1, n, rx2, ra1, ra2, phi1, A, phi2, v, nb, 0, 1, w.X, w.scale, nullptr, st);
-  forward_infer(nb, w.X, w.H1, w.H2, w.Y, st);
-  hipLaunchKernelGGL(scatter_kernel, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, st, rx1, n, rx2, w.Y, w.scale, z);
+  double* Ad = (double*)arena(kArenaMlp, sizeof(double) * 192 * (size_t)ra1 * ra2);
+  hipLaunchKernelGGL(diagonals_kernel, dim3((unsigned)(ra1 * ra2)), dim3(192), 0, st, n, ra1, ra2, A, Ad);
+  InferArgs a{};
+  a.ncols = nb;
+  a.w = g_model.wbf;
+  a.master = g_model.master;
+  a.rx1 = rx1; a.rx2 = rx2; a.ra1 = ra1; a.ra2 = ra2;
+  a.phi1 = phi1; a.Ad = Ad; a.phi2 = phi2; a.v = v; a.z = z;
+  hipLaunchKernelGGL(infer_kernel<true>, dim3((unsigned)((nb + kInfCols - 1) / kInfCols)), dim3(kInfThreads), 0, st,
+                     a);
   TTF_HIP(hipGetLastError());
 }
 
@@ -677,8 +758,15 @@ int ttf_mlp_forward(int M, const float* X, float* Y) {
     TTF_REQUIRE(g_model.ready, "ttf_mlp_forward: no parameters set");
     TTF_REQUIRE(M >= 0, "ttf_mlp_forward: M=%d", M);
     if (M == 0) return;
-    MlpWork w = work_for(M, false);
-    forward_infer(M, X, w.H1, w.H2, Y, stream());
+    InferArgs a{};
+    a.ncols = M;
+    a.w = g_model.wbf;
+    a.master = g_model.master;
+    a.X = X;
+    a.Y = Y;
+    hipLaunchKernelGGL(infer_kernel<false>, dim3((unsigned)(((int64_t)M + kInfCols - 1) / kInfCols)),
+                       dim3(kInfThreads), 0, stream(), a);
+    TTF_HIP(hipGetLastError());
   });
 }
 
@@ -687,7 +775,7 @@ int ttf_mlp_loss_grad(int M, const float* X, const float* T, double* loss, float
     TTF_REQUIRE(g_model.ready, "ttf_mlp_loss_grad: no parameters set");
     TTF_REQUIRE(M > 0, "ttf_mlp_loss_grad: M=%d", M);
     hipStream_t st = stream();
-    MlpWork w = work_for(M, true);
+    MlpWork w = work_for(M);
     float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * 2);
     double* out = (double*)(g + kMlpParams + (kMlpParams & 1));
     if ((reinterpret_cast<uintptr_t>(X) & 15) != 0) {
@@ -709,7 +797,7 @@ int ttf_mlp_train(long nsamples, const float* X, const float* T, int epochs, int
     hipStream_t st = stream();
     const int B = (int)std::min<long>(batch, nsamples);
     const long nbat = nsamples / B;
-    MlpWork w = work_for(B, true);
+    MlpWork w = work_for(B);
     float* g = (float*)arena(kArenaMlp2, sizeof(float) * (size_t)kMlpParams + sizeof(double) * (nbat + 1) +
                                              sizeof(int) * (size_t)nsamples + 64);
     double* losses = (double*)(g + kMlpParams + (kMlpParams & 1));
