@@ -33,7 +33,7 @@ CFLAGS = [
 SHARED_SOURCES = ["runtime.hip", "gemm.hip", "contract.hip", "linalg.hip", "lobpcg.hip", "eigb.hip",
                   "amen_local.hip", "amen.hip", "ksl.hip", "mlp.hip",
                   "eigb_batch.hip", "sdv_io.hip", "noalloc.hip", "mvk4.hip", "amen_typed.hip",
-                  "bfun3_fused.hip"]
+                  "bfun3_fused.hip", "bfun3_small.hip"]
 KIND_SOURCES = ["refabi.hip"]
 
 

@@ -1,0 +1,266 @@
+// The local matvec (ttals.f90:9-83) of small and middle ranks with narrow
+// modes in one launch, in all four element types:
+//   T1(b1,j,a2)  = sum_b2 x(b1,j,b2) phi2(b2,a2,c2)
+//   T2(b1,a1,i)  = sum_{j,a2} A(a1,i,j,a2) T1(b1,j,a2)
+//   y(c1,i,c2)   = sum_{b1,a1} phi1(c1,b1,a1) T2(b1,a1,i)
+// One work-group of eight waves per (vector, right-interface index c2), the
+// intermediates in LDS.  For one c2 the products have only ra2 and n
+// columns, which would fill a fraction of a 16-column matrix-core tile, and
+// the vector units multiply f64 at the matrix cores' rate: a thread keeps
+// one row's ra2 (or n) sums in registers, the narrow operand reaches all
+// lanes of a wave at once (phi2 by scalar loads, T2 by LDS broadcasts), and
+// the waves left over by the rows split the sum, their parts added in a
+// fixed order.
+#include "contract.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+
+namespace ttf {
+
+namespace {
+
+constexpr int kNT = 512;
+constexpr int kMaxCols = 8;          // ra2 and n at most
+constexpr int kInFlight = 8;         // loads of the wide operand per round trip
+constexpr size_t kLdsBytes = 96 * 1024;
+
+template <typename T>
+struct SmallArgs {
+  int rx1, m, rx2, ry1, n, ry2, ra1, ra2;
+  const T* phi1;
+  const T* A;      // nullptr: T2 = T1 (m = n = 1, ra1 = ra2)
+  const T* phi2;
+  const T* x;
+  int64_t ldx;
+  T* y;
+  int64_t ldy;
+};
+
+__device__ __forceinline__ double mac(double c, double a, double b) { return fma(a, b, c); }
+__device__ __forceinline__ float mac(float c, float a, float b) { return fmaf(a, b, c); }
+__device__ __forceinline__ hipDoubleComplex mac(hipDoubleComplex c, hipDoubleComplex a, hipDoubleComplex b) {
+  return make_hipDoubleComplex(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
+}
+__device__ __forceinline__ hipFloatComplex mac(hipFloatComplex c, hipFloatComplex a, hipFloatComplex b) {
+  return make_hipFloatComplex(fmaf(a.x, b.x, fmaf(-a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, c.y)));
+}
+__device__ __forceinline__ double plus(double a, double b) { return a + b; }
+__device__ __forceinline__ float plus(float a, float b) { return a + b; }
+__device__ __forceinline__ hipDoubleComplex plus(hipDoubleComplex a, hipDoubleComplex b) {
+  return make_hipDoubleComplex(a.x + b.x, a.y + b.y);
+}
+__device__ __forceinline__ hipFloatComplex plus(hipFloatComplex a, hipFloatComplex b) {
+  return make_hipFloatComplex(a.x + b.x, a.y + b.y);
+}
+template <typename T> __device__ __forceinline__ T zero() { return T(0); }
+template <> __device__ __forceinline__ hipDoubleComplex zero() { return make_hipDoubleComplex(0.0, 0.0); }
+template <> __device__ __forceinline__ hipFloatComplex zero() { return make_hipFloatComplex(0.f, 0.f); }
+
+// Threads per group of the rows x K split: whole waves, at most the block.
+__host__ __device__ inline int row_threads(int rows) {
+  const int r = (rows + 63) / 64 * 64;
+  return r < kNT ? r : kNT;
+}
+
+// part[(kg C + c) rows + r] = sum over group kg's share of k of W(r, k)
+// B(k, c), c < C, for the wide W (rows x K, ld rows, global) and the narrow
+// B given by at(k, c); groups of row_threads(rows) threads.
+template <int C, typename T, typename At>
+__device__ __forceinline__ void narrow_product(const T* __restrict__ W, int rows, int K, T* part, At at) {
+  const int rt = row_threads(rows), groups = kNT / rt;
+  const int kg = __builtin_amdgcn_readfirstlane((int)threadIdx.x / rt);
+  if (kg >= groups) return;   // uniform over the wave
+  const int per = (K + groups - 1) / groups;
+  const int k0 = kg * per, k1 = min(K, k0 + per);
+  for (int r = (int)threadIdx.x - kg * rt; r < (rows + rt - 1) / rt * rt; r += rt) {
+    const T* w = W + min(r, rows - 1);
+    T acc[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = zero<T>();
+    int k = k0;
+    for (; k + kInFlight <= k1; k += kInFlight) {
+      T v[kInFlight];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u) v[u] = w[(int64_t)rows * (k + u)];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[c] = mac(acc[c], v[u], at(k + u, c));
+    }
+    if (k < k1) {   // the rest, its loads clamped and its products skipped
+      T v[kInFlight];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u) v[u] = w[(int64_t)rows * min(k + u, k1 - 1)];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u)
+        if (k + u < k1) {   // uniform
+#pragma unroll
+          for (int c = 0; c < C; ++c) acc[c] = mac(acc[c], v[u], at(k + u, c));
+        }
+    }
+    if (r < rows) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) part[((int64_t)kg * C + c) * rows + r] = acc[c];
+    }
+  }
+}
+
+template <int C, typename T>
+__device__ __forceinline__ T group_sum(const T* part, int rows, int groups, int c, int r) {
+  T s = part[(int64_t)c * rows + r];
+  for (int g = 1; g < groups; ++g) s = plus(s, part[((int64_t)g * C + c) * rows + r]);
+  return s;
+}
+
+// A2 >= ra2 and N >= n columns; columns past them repeat the last one and
+// are dropped.
+template <typename T, int A2, int N>
+__global__ __launch_bounds__(kNT) void bfun3_small_kernel(SmallArgs<T> a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x;
+  const int c2 = blockIdx.x % a.ry2, v = blockIdx.x / a.ry2;
+  const int R1 = a.rx1 * a.m, K3 = a.rx1 * a.ra1;
+  T* T1 = reinterpret_cast<T*>(lds);       // (b1, j, a2)
+  T* T2 = T1 + R1 * a.ra2;                 // T2[(b1 + rx1 a1) N + i]
+  T* part = T2 + K3 * N;
+  {
+    const T* __restrict__ p2 = a.phi2 + (int64_t)a.rx2 * a.ra2 * c2;
+    const int rx2 = a.rx2, last = a.ra2 - 1;
+    narrow_product<A2>(a.x + v * a.ldx, R1, a.rx2, part,
+                       [&](int k, int c) { return p2[k + rx2 * (c < last ? c : last)]; });
+  }
+  __syncthreads();
+  {
+    const int groups = kNT / row_threads(R1);
+    for (int e = tid; e < R1 * a.ra2; e += kNT) {
+      const int c = e / R1;
+      T1[e] = group_sum<A2>(part, R1, groups, c, e - c * R1);
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < K3 * N; e += kNT) {
+    const int i = e / K3, k = e - i * K3;
+    T s = zero<T>();
+    if (i < a.n) {
+      if (a.A == nullptr) {
+        s = T1[k];
+      } else {
+        const int a1 = k / a.rx1, b1 = k - a1 * a.rx1;
+        const T* Ai = a.A + a1 + a.ra1 * i;
+        for (int q = 0; q < a.m * a.ra2; ++q) s = mac(s, Ai[(int64_t)a.ra1 * a.n * q], T1[b1 + a.rx1 * q]);
+      }
+    }
+    T2[k * N + i] = s;
+  }
+  __syncthreads();
+  narrow_product<N>(a.phi1, a.ry1, K3, part, [&](int k, int c) { return T2[k * N + c]; });
+  __syncthreads();
+  {
+    T* y = a.y + v * a.ldy + (int64_t)a.ry1 * a.n * c2;
+    const int groups = kNT / row_threads(a.ry1);
+    for (int e = tid; e < a.ry1 * a.n; e += kNT) {
+      const int i = e / a.ry1;
+      y[e] = group_sum<N>(part, a.ry1, groups, i, e - i * a.ry1);
+    }
+  }
+}
+
+int bucket(int c) { return c <= 2 ? 2 : c <= 3 ? 3 : c <= 5 ? 5 : 8; }
+
+template <typename T>
+size_t lds_need(const Shape& s, int A2, int N) {
+  const int64_t R1 = (int64_t)s.rx1 * s.m, K3 = (int64_t)s.rx1 * s.ra1;
+  const int64_t g1 = kNT / row_threads((int)std::min<int64_t>(R1, kNT)), g3 = kNT / row_threads(s.ry1);
+  return sizeof(T) * (size_t)(R1 * s.ra2 + K3 * N + std::max(g1 * A2 * R1, g3 * N * s.ry1));
+}
+
+bool small_enabled() {
+  static const bool on = [] {
+    const char* e = std::getenv("TTF_BFUN3_SMALL");
+    return !(e && std::atoi(e) == 0);
+  }();
+  return on;
+}
+
+// Where the one launch is the faster way: up to a number of multiply-adds
+// over all work-groups (columns as padded), past which the matrix cores'
+// tiles win.  Measured against the other path (us, other -> this), MPO rank
+// 5, n = 2, one vector unless said:
+//   f64   rank 2: 11.9 -> 4.7, 32: 13.7 -> 6.8, 64: 16.6 -> 8.6, 128: 29.1 ->
+//         18.8; 6 vectors at 64: 17.0 -> 12.7 (31e6), at 96: 26.0 -> 35.1
+//         (106e6); n = 4, rank 4, 6 vectors at 64: 16.2 -> 16.9 (63e6)
+//   f32   32: 15.5 -> 6.0, 128: 21.1 -> 13.7; 6 vectors at 96: 21.9 -> 20.1
+//         (106e6); n = 4, rank 4, 6 vectors at 96: 26.7 -> 27.0 (212e6)
+//   c128  32: 19.4 -> 7.6, 64: 21.8 -> 10.1, 128: 67.5 -> 24.5 (42e6); n = 4,
+//         rank 4 at 128: 61.0 -> 61.0 (84e6)
+//   c64   64: 17.9 -> 9.3, 128: 47.5 -> 22.5; n = 4, rank 4 at 128: 42.4 ->
+//         31.3 (84e6)
+template <typename T> constexpr double kMostMacs = 1.2e8;
+template <> constexpr double kMostMacs<double> = 5e7;
+template <> constexpr double kMostMacs<hipDoubleComplex> = 6e7;
+
+template <typename T>
+bool faster_small(const Shape& s, int nvec, int A2, int N) {
+  const double per = (double)s.rx1 * s.m * s.rx2 * A2 + (double)s.ry1 * s.rx1 * s.ra1 * N;
+  return per * s.ry2 * nvec <= kMostMacs<T>;
+}
+
+template <typename T, int A2, int N>
+void launch_n(const SmallArgs<T>& a, unsigned grid, size_t lds, hipStream_t st) {
+  static std::atomic<bool> attr{false};   // concurrent first calls only repeat the call
+  if (!attr) {
+    TTF_HIP(hipFuncSetAttribute((const void*)bfun3_small_kernel<T, A2, N>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+    attr = true;
+  }
+  hipLaunchKernelGGL((bfun3_small_kernel<T, A2, N>), dim3(grid), dim3(kNT), lds, st, a);
+}
+
+template <typename T, int A2>
+void launch(const SmallArgs<T>& a, int N, unsigned grid, size_t lds, hipStream_t st) {
+  switch (N) {
+    case 2: launch_n<T, A2, 2>(a, grid, lds, st); break;
+    case 3: launch_n<T, A2, 3>(a, grid, lds, st); break;
+    case 5: launch_n<T, A2, 5>(a, grid, lds, st); break;
+    default: launch_n<T, A2, 8>(a, grid, lds, st); break;
+  }
+}
+
+}  // namespace
+
+template <typename T>
+bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
+                 int64_t ldy, hipStream_t st) {
+  if (!small_enabled() || nvec < 1 || s.ra2 > kMaxCols || s.n > kMaxCols) return false;
+  const int64_t R1 = (int64_t)s.rx1 * s.m, K3 = (int64_t)s.rx1 * s.ra1;
+  if (R1 > 2048 || K3 > 4096 || s.ry1 > 2048) return false;
+  const int A2 = bucket(s.ra2), N = bucket(s.n);
+  if (!faster_small<T>(s, nvec, A2, N)) return false;
+  const size_t lds = lds_need<T>(s, A2, N);
+  if (lds > kLdsBytes || (int64_t)s.ry2 * nvec > 0x7fffffff / kNT) return false;
+  SmallArgs<T> a{s.rx1, s.m, s.rx2, s.ry1, s.n, s.ry2, s.ra1, s.ra2, phi1, A, phi2, x, ldx, y, ldy};
+  const unsigned grid = (unsigned)(s.ry2 * nvec);
+  switch (A2) {
+    case 2: launch<T, 2>(a, N, grid, lds, st); break;
+    case 3: launch<T, 3>(a, N, grid, lds, st); break;
+    case 5: launch<T, 5>(a, N, grid, lds, st); break;
+    default: launch<T, 8>(a, N, grid, lds, st); break;
+  }
+  TTF_HIP(hipGetLastError());
+  return true;
+}
+
+template bool bfun3_small<double>(const Shape&, int, const double*, const double*, const double*, const double*,
+                                  int64_t, double*, int64_t, hipStream_t);
+template bool bfun3_small<float>(const Shape&, int, const float*, const float*, const float*, const float*, int64_t,
+                                 float*, int64_t, hipStream_t);
+template bool bfun3_small<hipDoubleComplex>(const Shape&, int, const hipDoubleComplex*, const hipDoubleComplex*,
+                                            const hipDoubleComplex*, const hipDoubleComplex*, int64_t,
+                                            hipDoubleComplex*, int64_t, hipStream_t);
+template bool bfun3_small<hipFloatComplex>(const Shape&, int, const hipFloatComplex*, const hipFloatComplex*,
+                                           const hipFloatComplex*, const hipFloatComplex*, int64_t,
+                                           hipFloatComplex*, int64_t, hipStream_t);
+
+}  // namespace ttf

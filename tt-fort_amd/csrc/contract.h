@@ -27,6 +27,15 @@ bool bfun3_fused(const Shape& s, int nvec, const double* phi1, const double* A, 
                  const double* x, int64_t ldx, double* y, int64_t ldy, hipStream_t st);
 bool bfun3_fused_fits(const Shape& s, int nvec);
 
+// The whole chain in one launch on the vector units (bfun3_small.hip), for
+// narrow modes and operator ranks (n, ra2 <= 8) at the sizes where that is
+// the faster way, unless TTF_BFUN3_SMALL is 0; false leaves y untouched.
+// A == nullptr stands for the identity (m = n = 1, ra1 = ra2).  x and y must
+// not overlap.  T: double, float, hipDoubleComplex, hipFloatComplex.
+template <typename T>
+bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
+                 int64_t ldy, hipStream_t st);
+
 template <typename T>
 void bfun3_chain(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x,
                  int64_t ldx, T* y, int64_t ldy, hipStream_t st);

@@ -63,11 +63,12 @@ void bfun3_stage12(const Shape& s, int nvec, const T* A, const T* phi2, const T*
   gemm_launch(bfun3_op2(s, nvec, A, (const T*)T1, T2), st);
 }
 
-// true when the column blocks [x, x + ldx nvec) and [y, y + ldy nvec) overlap
+// true when the nvec columns of x and of y (leading dimensions ldx, ldy;
+// those of a single column are not used) overlap in memory
 template <typename T>
-static bool overlaps(const T* x, int64_t ldx, const T* y, int64_t ldy, int nvec) {
-  const T* xe = x + ldx * nvec;
-  const T* ye = y + ldy * nvec;
+static bool overlaps(const Shape& s, const T* x, int64_t ldx, const T* y, int64_t ldy, int nvec) {
+  const T* xe = x + ldx * (nvec - 1) + (int64_t)s.rx1 * s.m * s.rx2;
+  const T* ye = y + ldy * (nvec - 1) + (int64_t)s.ry1 * s.n * s.ry2;
   return x < ye && y < xe;
 }
 
@@ -75,8 +76,10 @@ template <typename T>
 void bfun3_chain(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x,
                  int64_t ldx, T* y, int64_t ldy, hipStream_t st) {
   if (nvec <= 0) return;
-  if constexpr (std::is_same<T, double>::value) {
-    if (!overlaps(x, ldx, y, ldy, nvec) && bfun3_fused(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
+  if (!overlaps(s, x, ldx, y, ldy, nvec)) {
+    if (bfun3_small(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
+    if constexpr (std::is_same<T, double>::value)
+      if (bfun3_fused(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
   }
   const int64_t sz1 = (int64_t)s.rx1 * s.m * s.ra2 * s.ry2;
   const int64_t sz2 = (int64_t)s.rx1 * s.ra1 * s.n * s.ry2;
@@ -102,9 +105,11 @@ template <typename T>
 void bfun3_chain_ws(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x,
                     int64_t ldx, T* y, int64_t ldy, T* ws, size_t ws_cap, hipStream_t st) {
   if (nvec <= 0) return;
-  // the fused kernel keeps its intermediates in LDS and allocates nothing
-  if constexpr (std::is_same<T, double>::value) {
-    if (!overlaps(x, ldx, y, ldy, nvec) && bfun3_fused(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
+  // the one-launch kernels keep their intermediates in LDS and allocate nothing
+  if (!overlaps(s, x, ldx, y, ldy, nvec)) {
+    if (bfun3_small(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
+    if constexpr (std::is_same<T, double>::value)
+      if (bfun3_fused(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st)) return;
   }
   const size_t need = bfun3_workspace(s, nvec);
   TTF_REQUIRE(ws != nullptr && need <= ws_cap, "bfun3: workspace of %zu elements exceeds the %zu given", need,
@@ -155,6 +160,9 @@ static void zbfun3_chain_t(const Shape& s, int nvec, const typename CplxT<R>::ty
                            hipStream_t st) {
   typedef typename CplxT<R>::type C_t;
   if (nvec <= 0) return;
+  if (!overlaps(s, (const C_t*)x, ldx, (const C_t*)y, ldy, nvec) &&
+      bfun3_small<C_t>(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st))
+    return;
   const int64_t sz1 = (int64_t)s.rx1 * s.m * s.ra2 * s.ry2;
   const int64_t sz2 = (int64_t)s.rx1 * s.ra1 * s.n * s.ry2;
   C_t* T1 = (C_t*)arena(kArenaBfun, sizeof(C_t) * (size_t)(sz1 + sz2) * nvec);
@@ -575,7 +583,7 @@ int ttf_dbfun3_chain_profile(int rx1, int m, int rx2, int ry1, int n, int ry2, i
     Shape s = mkshape(rx1, m, rx2, ry1, n, ry2, ra1, ra2);
     TTF_REQUIRE(iters > 0 && nvec > 0 && ms != nullptr, "ttf_dbfun3_chain_profile: bad arguments");
     hipStream_t st = stream();
-    if (fused) *fused = bfun3_fused_fits(s, nvec) && !overlaps(x, ldx, (const double*)y, ldy, nvec) ? 1 : 0;
+    if (fused) *fused = bfun3_fused_fits(s, nvec) && !overlaps(s, x, ldx, (const double*)y, ldy, nvec) ? 1 : 0;
     bfun3_chain<double>(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st);   // settles any tuning
     hipEvent_t e0, e1;
     TTF_HIP(hipEventCreate(&e0));

@@ -1031,6 +1031,9 @@ struct SOp {
   const zc* phi2;
   zc* work;   // rx1 * ra * ry2
   void apply(const zc* Sx, zc* Sy, hipStream_t st) const {
+    // the local matvec without a core: modes of 1 and the identity between
+    const Shape s{rx1, 1, rx2, ry1, 1, ry2, ra, ra};
+    if (bfun3_small<zc>(s, 1, phi1, nullptr, phi2, Sx, 0, Sy, 0, st)) return;
     const zc one{1.0, 0.0}, zero{0.0, 0.0};
     zgemm_cm('N', 'N', rx1, ra * ry2, rx2, one, Sx, rx1, phi2, rx2, zero, work, rx1, st);
     zgemm_cm('N', 'N', ry1, ry2, rx1 * ra, one, phi1, ry1, work, rx1 * ra, zero, Sy, ry1, st);
