@@ -225,62 +225,72 @@ static Cfg heuristic(int M, int N, int K, int nbatch) {
   return {best->bm, best->bn, ks};
 }
 
-template <typename T, bool CT, bool VEC>
+template <typename T, bool CT, int MODE>
 static void launch_tiles(const GemmOp<T>& op, const Cfg& c, hipStream_t st) {
   const unsigned wgs = (unsigned)(ceil_div(op.M, c.bm) * ceil_div(op.N, c.bn) * op.nbatch * op.ksplit);
   // K chunk: 16 for f64, 32 for f32 (a 16-byte load covers four k); the
   // small tiles, latency-bound on each chunk, take twice as much
-  constexpr int BK = sizeof(T) == 8 ? 16 : 32, BK1 = VEC ? 2 * BK : BK;
+  constexpr int BK = sizeof(T) == 8 ? 16 : 32, BK1 = MODE == kVecBoth ? 2 * BK : BK;
   switch (1000 * c.bm + c.bn) {
     case 128064:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 64, BK, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 64, BK, 2, 2, CT, MODE>), dim3(wgs), dim3(256), 0, st, op);
       break;
     case 64096:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 96, BK, 4, 2, CT, VEC>), dim3(wgs), dim3(512), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 96, BK, 4, 2, CT, MODE>), dim3(wgs), dim3(512), 0, st, op);
       break;
     case 64080:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 80, BK, 4, 1, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 80, BK, 4, 1, CT, MODE>), dim3(wgs), dim3(256), 0, st, op);
       break;
     case 64064:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, BK, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, BK, 2, 2, CT, MODE>), dim3(wgs), dim3(256), 0, st, op);
       break;
     case 64032:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 32, BK, 4, 1, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 32, BK, 4, 1, CT, MODE>), dim3(wgs), dim3(256), 0, st, op);
       break;
     case 32032:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, BK1, 2, 2, CT, VEC>), dim3(wgs), dim3(256), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 32, BK1, 2, 2, CT, MODE>), dim3(wgs), dim3(256), 0, st, op);
       break;
     default:
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, BK1, 1, 1, CT, VEC>), dim3(wgs), dim3(64), 0, st, op);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 32, 16, BK1, 1, 1, CT, MODE>), dim3(wgs), dim3(64), 0, st, op);
       break;
   }
 }
 
+// Whether an operand's offsets inside a tile (at most 128 rows and 64 of k)
+// fit 32 bits.
+template <typename T>
+static bool operand_near(int64_t s_row, int64_t s_k) {
+  const int64_t most = ((int64_t)1 << 32) / (int64_t)sizeof(T);
+  return s_row >= 0 && s_k >= 0 && s_row < most && s_k < most && 128 * s_row + 64 * s_k < most;
+}
+
 // Whether an operand (rows x K, strides s_row, s_k, batch strides) can be
 // read 16 bytes at a time along its contiguous direction: pointer, other
-// strides and the extent of that direction all whole multiples of 16 bytes,
-// and a tile's offsets (at most 128 rows or 64 of k) below 2^32 bytes.
+// strides and the extent of that direction all whole multiples of 16 bytes.
 template <typename T>
 static bool operand_aligned(const T* p, int64_t s_row, int64_t s_k, int64_t sb0, int64_t sb1, int rows, int K) {
   constexpr int V = 16 / (int)sizeof(T);
   if ((reinterpret_cast<uintptr_t>(p) & 15) != 0 || sb0 % V != 0 || sb1 % V != 0) return false;
-  const int64_t reach = (int64_t)1 << 22;   // elements: 127 rows of it are below 2^32 bytes
-  if (s_row == 1) return s_k % V == 0 && rows % V == 0 && s_k > 0 && s_k < reach;
-  return s_k == 1 && s_row % V == 0 && K % V == 0 && s_row > 0 && s_row < reach;
+  if (s_row == 1) return s_k % V == 0 && rows % V == 0;
+  return s_k == 1 && s_row % V == 0 && K % V == 0;
 }
 
 template <typename T>
 static void launch_cfg(GemmOp<T> op, const Cfg& c, hipStream_t st) {
   op.ksplit = c.ks;
-  const bool vec = operand_aligned(op.A, op.sAi, op.sAk, op.sAb0, op.sAb1, op.M, op.K) &&
-                   operand_aligned(op.B, op.sBj, op.sBk, op.sBb0, op.sBb1, op.N, op.K);
   // column-contiguous outputs (and the column-major split-K slices) take the
-  // swapped-fragment variant, whose lanes store consecutive rows
+  // swapped-fragment variant, whose lanes store consecutive rows; the other
+  // outputs are few, and small, and read element by element
   const bool ct = op.ksplit > 1 || op.sCi == 1;
-  if (ct && vec) launch_tiles<T, true, true>(op, c, st);
-  else if (ct) launch_tiles<T, true, false>(op, c, st);
-  else if (vec) launch_tiles<T, false, true>(op, c, st);
-  else launch_tiles<T, false, false>(op, c, st);
+  const bool near = operand_near<T>(op.sAi, op.sAk) && operand_near<T>(op.sBj, op.sBk);
+  const bool va = operand_aligned(op.A, op.sAi, op.sAk, op.sAb0, op.sAb1, op.M, op.K);
+  const bool vb = operand_aligned(op.B, op.sBj, op.sBk, op.sBb0, op.sBb1, op.N, op.K);
+  if (!ct) launch_tiles<T, false, kWide>(op, c, st);
+  else if (!near) launch_tiles<T, true, kWide>(op, c, st);
+  else if (va && vb) launch_tiles<T, true, kVecBoth>(op, c, st);
+  else if (va) launch_tiles<T, true, kVecA>(op, c, st);
+  else if (vb) launch_tiles<T, true, kVecB>(op, c, st);
+  else launch_tiles<T, true, kScalar>(op, c, st);
   TTF_HIP(hipGetLastError());
   if (op.ksplit > 1) {
     int64_t total = (int64_t)op.M * op.N * op.nbatch;

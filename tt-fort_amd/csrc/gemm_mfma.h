@@ -90,15 +90,20 @@ __device__ __forceinline__ int xcd_remap(int wg, int total) {
 // (44 -> 57 TFLOP/s; a large product reaches 72 here); rank 64, n 64,
 // operator rank 6, one vector 67.5 -> 52.5 us in f64 and 53.9 -> 41.8 us in
 // f32 at ranks 61 and 57.  The next chunk is loaded to registers while the current one
-// is multiplied out of one of two LDS buffers (one barrier per chunk).  With
-// VEC, operands move 16 bytes per lane along their contiguous direction (the
-// launcher checks the alignment of pointers, strides and extents).
+// is multiplied out of one of two LDS buffers (one barrier per chunk).  The
+// launcher picks the widest loads that the operands' alignment allows.
 //
 // CT (column-contiguous output, op.sCi == 1): the fragments are multiplied
 // in swapped order, B^T A^T, so that each accumulator holds a tile of C^T:
 // lane l then owns row l%16 of the 16x16 block and consecutive lanes store
 // consecutive rows (contiguous in memory) instead of consecutive columns.
 template <typename T, int V> struct VecOf;
+// How a tile reads its operands: 16 bytes per lane along the contiguous
+// direction where pointer, strides and extents allow it, else element by
+// element, each operand for itself; kWide: element by element with 64-bit
+// offsets.
+enum LoadMode { kWide, kScalar, kVecA, kVecB, kVecBoth };
+
 template <> struct VecOf<double, 2> { typedef double type __attribute__((ext_vector_type(2))); };
 template <> struct VecOf<float, 4> { typedef float type __attribute__((ext_vector_type(4))); };
 template <typename T> struct VecOf<T, 1> { typedef T type __attribute__((ext_vector_type(1))); };
@@ -106,7 +111,7 @@ template <typename T> struct VecOf<T, 1> { typedef T type __attribute__((ext_vec
 // One operand's tile loader: R rows (or columns) x BK of k, V elements per
 // load along the contiguous direction (`along_k`: that direction is k).
 // Thread t takes the vectors t, t + NT, ...
-template <typename T, int R, int BK, int NT, int V>
+template <typename T, int R, int BK, int NT, int V, bool WIDE>
 struct TileLoad {
   typedef typename VecOf<T, V>::type vec_t;
   static constexpr int TOTAL = R * BK / V;
@@ -114,12 +119,13 @@ struct TileLoad {
   static constexpr bool EVEN = TOTAL % NT == 0;
   static constexpr int PAD = 16 / (int)sizeof(T);   // keeps 16-byte LDS rows
 
-  // With V > 1 (where the launcher has checked that they fit) each vector is
-  // at a 32-bit offset from a uniform base, so that moving to the next chunk
-  // costs no vector instructions; else it has a pointer of its own.
+  // Each vector is at a 32-bit offset from a uniform base, so that moving to
+  // the next chunk costs no vector instructions; with WIDE (strides whose
+  // offsets do not fit) it has a pointer of its own.
+  static_assert(!WIDE || V == 1, "wide strides are read element by element");
   const T* base;
-  unsigned off[V > 1 ? L : 1];
-  const T* p[V > 1 ? 1 : L];
+  unsigned off[WIDE ? 1 : L];
+  const T* p[WIDE ? L : 1];
   int lds[L];        // LDS positions, k * (R + PAD) + row
   vec_t v[L];
   int64_t step;      // advance per chunk
@@ -145,14 +151,14 @@ struct TileLoad {
       int row, k;
       split(threadIdx.x + q * NT, along_k, &row, &k);
       lds[q] = k * (R + PAD) + row;
-      if constexpr (V > 1) off[q] = (unsigned)(sizeof(T) * (s_row * min(row, last) + s_k * k));
+      if constexpr (!WIDE) off[q] = (unsigned)(sizeof(T) * (s_row * min(row, last) + s_k * k));
       else p[q] = base + s_row * min(row, last) + s_k * k;
     }
   }
   __device__ __forceinline__ void load() {
 #pragma unroll
     for (int q = 0; q < L; ++q) {
-      if constexpr (V > 1) {
+      if constexpr (!WIDE) {
         v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base) + off[q]);
       } else {
         v[q][0] = *p[q];
@@ -168,7 +174,7 @@ struct TileLoad {
       int row, k;
       split(threadIdx.x + q * NT, along_k, &row, &k);
       const int64_t back = sk * (min(k, along_k ? left - V : left - 1) - k);
-      if constexpr (V > 1)
+      if constexpr (!WIDE)
         v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base + back) + off[q]);
       else
         v[q][0] = p[q][back];
@@ -209,18 +215,19 @@ struct TileLoad {
 // operand's extent).  With FOLD each chunk's products are summed by
 // themselves and then added, which shortens the rounding chain of long f32
 // sums.
-template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC, bool FOLD = false>
+template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, int MODE, bool FOLD = false>
 struct GemmTile {
   static constexpr int NT = 64 * WR * WC;
-  static constexpr int V = VEC ? 16 / (int)sizeof(T) : 1;
+  static constexpr int VA = MODE == kVecA || MODE == kVecBoth ? 16 / (int)sizeof(T) : 1;
+  static constexpr int VB = MODE == kVecB || MODE == kVecBoth ? 16 / (int)sizeof(T) : 1;
   static constexpr int WM = BM / WR, WN = BN / WC;
   static constexpr int FM = WM / 16, FN = WN / 16;
   static_assert(FM * 16 * WR == BM && FN * 16 * WC == BN, "wave tiles of whole fragments");
   typedef typename Acc4<T>::type acc_t;
-  typedef TileLoad<T, BM, BK, NT, V> LoadA;
-  typedef TileLoad<T, BN, BK, NT, V> LoadB;
+  typedef TileLoad<T, BM, BK, NT, VA, MODE == kWide> LoadA;
+  typedef TileLoad<T, BN, BK, NT, VB, MODE == kWide> LoadB;
   static constexpr int LDA = BM + LoadA::PAD, LDB = BN + LoadB::PAD;
-  static_assert(V == 1 || (LDA * sizeof(T) % 16 == 0 && LDB * sizeof(T) % 16 == 0), "LDS rows of whole 16 bytes");
+  static_assert(LDA * sizeof(T) % 16 == 0 && LDB * sizeof(T) % 16 == 0, "LDS rows of whole 16 bytes");
 
   acc_t acc[FM][FN];
 
@@ -309,9 +316,9 @@ struct GemmTile {
   }
 };
 
-template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, bool VEC>
+template <typename T, int BM, int BN, int BK, int WR, int WC, bool CT, int MODE>
 __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_mfma_kernel(GemmOp<T> op) {
-  typedef GemmTile<T, BM, BN, BK, WR, WC, CT, VEC> Tile;
+  typedef GemmTile<T, BM, BN, BK, WR, WC, CT, MODE> Tile;
   constexpr int FM = Tile::FM, FN = Tile::FN;
   // consecutive logical tiles share an XCD and so an L2; they go down bands
   // of eight tile rows, so that the tiles in flight on an XCD read about as

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void features_kernel(int rx1, int n, int rx2, 
 // (the output layer): the point-Jacobi term X0(3 kMlpBlock + n, m) /
 // X0(n, m) of the input features X0 is added, Y = dL/dY = f (y - T) with the
 // targets T, and part[work-group] = the sum of (y - T)^2.
-typedef GemmTile<float, 32, 32, 64, 2, 2, true, true, true> LayerTile;
+typedef GemmTile<float, 32, 32, 64, 2, 2, true, kVecBoth> LayerTile;
 
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void train_layer_kernel(GemmOp<float> op, const float* __restrict__ bias,
@@ -191,22 +191,27 @@ __global__ __launch_bounds__(256, 2) void train_layer_kernel(GemmOp<float> op, c
   }
 }
 
+// The backward sums are folded per chunk of 64 (the split sums that they
+// replace were); the forward ones stay one chain, so that the loss keeps its
+// bits.
+typedef GemmTile<float, 32, 32, 64, 2, 2, true, kVecBoth, true> BackTile;
+
 // dH (kMlpHid x M) = W D with the ReLU derivative from the activation H
 // itself: zero where H is not positive.
 __global__ __launch_bounds__(256, 2) void train_back_kernel(GemmOp<float> op, const float* __restrict__ H) {
   const int tilesN = (op.N + 31) / 32;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int tm = wg / tilesN, tn = wg - tm * tilesN;
-  LayerTile t;
+  BackTile t;
   t.sums(op, op.A, op.B, tm * 32, tn * 32, 0, op.K);
   float h[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r)
-    h[r] = H[min(tm * 32 + LayerTile::row(0, r), op.M - 1) +
-             (int64_t)op.M * min(tn * 32 + LayerTile::col(0, r), op.N - 1)];
+    h[r] = H[min(tm * 32 + BackTile::row(0, r), op.M - 1) +
+             (int64_t)op.M * min(tn * 32 + BackTile::col(0, r), op.N - 1)];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int n = tm * 32 + LayerTile::row(0, r), m = tn * 32 + LayerTile::col(0, r);
+    const int n = tm * 32 + BackTile::row(0, r), m = tn * 32 + BackTile::col(0, r);
     if (n < op.M && m < op.N) op.C[n + (int64_t)op.M * m] = h[r] > 0.f ? t.acc[0][0][r] : 0.f;
   }
 }
@@ -219,7 +224,7 @@ constexpr int kGradSlices = 16;
 constexpr int kGradTiles = 4 * (kMlpHid + kMlpHid + kMlpOut) / 64;   // 36 weight tiles
 constexpr int kGradRows = (kMlpHid + kMlpHid + kMlpOut) / 64;        // 9 bias groups
 static_assert(kMlpIn == 256 && kMlpHid == 256 && kMlpOut == 64, "gradient tiles");
-typedef GemmTile<float, 64, 64, 32, 2, 2, true, true, true> GradTile;
+typedef GemmTile<float, 64, 64, 32, 2, 2, true, kVecBoth, true> GradTile;
 
 struct WeightGrads {
   const float* in[3];   // X, H1, H2 (256 x M)
