@@ -89,8 +89,10 @@ __device__ __forceinline__ int xcd_remap(int wg, int total) {
 // local matvecs: rank 512, n 2, MPO rank 5, 8 vectors, f64 983 -> 761 us
 // (44 -> 57 TFLOP/s; a large product reaches 72 here); rank 64, n 64,
 // operator rank 6, one vector 67.5 -> 52.5 us in f64 and 53.9 -> 41.8 us in
-// f32 at ranks 61 and 57.  The next chunk is loaded to registers while the current one
-// is multiplied out of one of two LDS buffers (one barrier per chunk).  The
+// f32 at ranks 61 and 57.  The next two chunks are on their way to registers while
+// the current one is multiplied out of one of two LDS buffers (one barrier
+// per chunk): an operand that the previous kernel wrote comes from another
+// XCD's cache, and one chunk's products do not cover that way.  The
 // launcher picks the widest loads that the operands' alignment allows.
 //
 // CT (column-contiguous output, op.sCi == 1): the fragments are multiplied
@@ -127,7 +129,7 @@ struct TileLoad {
   unsigned off[WIDE ? 1 : L];
   const T* p[WIDE ? L : 1];
   int lds[L];        // LDS positions, k * (R + PAD) + row
-  vec_t v[L];
+  vec_t v[2][L];     // two chunks in flight
   int64_t step;      // advance per chunk
   int64_t sk;
   bool along_k;
@@ -155,49 +157,49 @@ struct TileLoad {
       else p[q] = base + s_row * min(row, last) + s_k * k;
     }
   }
-  __device__ __forceinline__ void load() {
+  __device__ __forceinline__ void load(int set) {
 #pragma unroll
     for (int q = 0; q < L; ++q) {
       if constexpr (!WIDE) {
-        v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base) + off[q]);
+        v[set][q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base) + off[q]);
       } else {
-        v[q][0] = *p[q];
+        v[set][q][0] = *p[q];
         p[q] += step;
       }
     }
     base += step;
   }
   // the chunk that crosses the end of K: `left` = valid k of the chunk
-  __device__ __forceinline__ void load_tail(int left) {
+  __device__ __forceinline__ void load_tail(int left, int set) {
 #pragma unroll
     for (int q = 0; q < L; ++q) {
       int row, k;
       split(threadIdx.x + q * NT, along_k, &row, &k);
       const int64_t back = sk * (min(k, along_k ? left - V : left - 1) - k);
       if constexpr (!WIDE)
-        v[q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base + back) + off[q]);
+        v[set][q] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const char*>(base + back) + off[q]);
       else
-        v[q][0] = p[q][back];
+        v[set][q][0] = p[q][back];
     }
 #pragma unroll
     for (int q = 0; q < L; ++q) {
       int row, k;
       split(threadIdx.x + q * NT, along_k, &row, &k);
 #pragma unroll
-      for (int u = 0; u < V; ++u) v[q][u] = k < left ? v[q][u] : T(0);
+      for (int u = 0; u < V; ++u) v[set][q][u] = k < left ? v[set][q][u] : T(0);
     }
   }
-  __device__ __forceinline__ void store(T* s) const {
+  __device__ __forceinline__ void store(T* s, int set) const {
     if (V > 1 && !along_k) {
 #pragma unroll
       for (int q = 0; q < L; ++q)
-        if (EVEN || (int)threadIdx.x + q * NT < TOTAL) *reinterpret_cast<vec_t*>(s + lds[q]) = v[q];
+        if (EVEN || (int)threadIdx.x + q * NT < TOTAL) *reinterpret_cast<vec_t*>(s + lds[q]) = v[set][q];
     } else {
 #pragma unroll
       for (int q = 0; q < L; ++q)
         if (EVEN || (int)threadIdx.x + q * NT < TOTAL) {
 #pragma unroll
-          for (int u = 0; u < V; ++u) s[lds[q] + u * (R + PAD)] = v[q][u];
+          for (int u = 0; u < V; ++u) s[lds[q] + u * (R + PAD)] = v[set][q][u];
         }
     }
   }
@@ -256,15 +258,19 @@ struct GemmTile {
     LoadB lb;
     la.init(A, op.sAi, op.sAk, row0, op.M, kbeg);
     lb.init(B, op.sBj, op.sBk, col0, op.N, kbeg);
-    auto load = [&](int c) {
+    auto load = [&](int c, int set) {
       const int left = kend - kbeg - c * BK;
       if (left >= BK) {
-        la.load();
-        lb.load();
+        la.load(set);
+        lb.load(set);
       } else {
-        la.load_tail(left);
-        lb.load_tail(left);
+        la.load_tail(left, set);
+        lb.load_tail(left, set);
       }
+    };
+    auto store = [&](int buf, int set) {
+      la.store(As[buf], set);
+      lb.store(Bs[buf], set);
     };
     const int arow = (lane >> 4) * LDA + wm * WM + (lane & 15);
     const int brow = (lane >> 4) * LDB + wn * WN + (lane & 15);
@@ -299,20 +305,23 @@ struct GemmTile {
           for (int j = 0; j < FN; ++j) acc[i][j] += own[i][j];
       }
     };
-    load(0);
-    la.store(As[0]);
-    lb.store(Bs[0]);
+    load(0, 0);
+    if (nch > 1) load(1, 1);
+    store(0, 0);
     __syncthreads();
-    // one exit, after the last chunk but one: a second way out of the loop
-    // makes the compiler copy every accumulator in each turn
-    for (int c = 0; c < nch - 1; ++c) {
-      load(c + 1);
-      multiply(c & 1);
-      la.store(As[(c + 1) & 1]);
-      lb.store(Bs[(c + 1) & 1]);
+    // two chunks a turn, one exit: a second way out of the loop makes the
+    // compiler copy every accumulator in each turn
+    for (int c = 0; c + 1 < nch; c += 2) {
+      if (c + 2 < nch) load(c + 2, 0);
+      multiply(0);
+      store(1, 1);
+      __syncthreads();
+      if (c + 3 < nch) load(c + 3, 1);
+      multiply(1);
+      if (c + 2 < nch) store(0, 0);
       __syncthreads();
     }
-    multiply((nch - 1) & 1);
+    if (nch & 1) multiply(0);
   }
 };
 
