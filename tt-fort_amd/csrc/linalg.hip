@@ -664,6 +664,201 @@ __global__ __launch_bounds__(256) void qr_panel_kernel(int rows, int pc, double*
     for (int i = tid; i < rows; i += blockDim.x) Yb[i + (int64_t)rows * c] = P[c * lp + i];
 }
 
+// The same panel factorisation with the columns in registers, for panels of
+// up to 64 NRL rows and 32 columns: sixteen waves, two columns each, lane l
+// holding rows l, l + 64, ...  A step is a chain of latencies (norm,
+// reflector, dot products, update), so it is kept short: the owning wave
+// forms the reflector from its own registers, one LDS copy of it and one
+// barrier later every wave projects its columns, and the dot products of the
+// reflector with the earlier ones, which T needs, fall out of the same
+// instructions.  640 rows: 121 us a panel of 25 columns (all an LDS-resident
+// panel holds) -> 61 to 71 us a panel of 32.
+constexpr int kQrWaves = kQrPanel / 2;
+constexpr int kQrChunk = 256;   // rows of V staged at a time for Y
+
+template <int NRL>
+__global__ __launch_bounds__(64 * kQrWaves) void qr_panel_reg_kernel(int rows, int pc, double* __restrict__ X,
+                                                                     int64_t ld, double* __restrict__ Vb,
+                                                                     double* __restrict__ Yb, int64_t sX,
+                                                                     int64_t sVY) {
+  extern __shared__ double lds[];
+  X += blockIdx.y * sX;
+  Vb += blockIdx.y * sVY;
+  Yb += blockIdx.y * sVY;
+  double* vbuf = lds;                                // the reflector, double-buffered: 2 x 64 NRL
+  double* P = lds;                                   // V by chunks afterwards: column c at c (kQrChunk + 1)
+  __shared__ double S[kQrPanel][kQrPanel + 1], T[kQrPanel][kQrPanel + 1];
+  __shared__ double tau[kQrPanel];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int e = tid; e < kQrPanel * (kQrPanel + 1); e += 64 * kQrWaves) {
+    (&S[0][0])[e] = 0.0;
+    (&T[0][0])[e] = 0.0;
+  }
+  __syncthreads();
+  double a0[NRL], a1[NRL];   // this wave's columns 2 wave, 2 wave + 1
+  {
+    const int c0 = min(2 * wave, pc - 1), c1 = min(2 * wave + 1, pc - 1);
+#pragma unroll
+    for (int t = 0; t < NRL; ++t) {
+      const int r = min(lane + 64 * t, rows - 1);
+      a0[t] = X[r + ld * c0];
+      a1[t] = X[r + ld * c1];
+    }
+#pragma unroll
+    for (int t = 0; t < NRL; ++t) {
+      const bool in = lane + 64 * t < rows;
+      a0[t] = in && 2 * wave < pc ? a0[t] : 0.0;
+      a1[t] = in && 2 * wave + 1 < pc ? a1[t] : 0.0;
+    }
+  }
+  for (int j = 0; j < pc; ++j) {
+    double* vb = vbuf + (j & 1) * 64 * NRL;
+    if (wave == (j >> 1)) {   // uniform
+      const bool second = j & 1;
+      double x[NRL], s = 0.0;
+#pragma unroll
+      for (int t = 0; t < NRL; ++t) {
+        x[t] = second ? a1[t] : a0[t];
+        if (t > 0 || lane > j) s += x[t] * x[t];   // j < 32: rows past j are lanes past j of the first slab
+      }
+      s = wave_sum64(s);
+      const double x0 = readlane_f64(x[0], j);   // zero when j >= rows
+      double tj = 0.0, beta = x0, scal = 0.0;
+      if (s > 0.0) {
+        const double nrm = sqrt(x0 * x0 + s);
+        beta = x0 >= 0.0 ? -nrm : nrm;
+        tj = (beta - x0) / beta;
+        scal = 1.0 / (x0 - beta);
+      }
+      if (lane == 0) tau[j] = tj;
+#pragma unroll
+      for (int t = 0; t < NRL; ++t) {
+        const bool below = t > 0 || lane > j, diag = t == 0 && lane == j;
+        const double y = x[t] * scal;
+        vb[lane + 64 * t] = below ? y : (diag ? 1.0 : 0.0);
+        const double keep = below ? y : (diag ? beta : x[t]);
+        a0[t] = second ? a0[t] : keep;
+        a1[t] = second ? keep : a1[t];
+      }
+    }
+    __syncthreads();
+    double v[NRL], w0 = 0.0, w1 = 0.0;
+#pragma unroll
+    for (int t = 0; t < NRL; ++t) v[t] = vb[lane + 64 * t];
+#pragma unroll
+    for (int t = 0; t < NRL; ++t) {
+      w0 += a0[t] * v[t];
+      w1 += a1[t] * v[t];
+    }
+    w0 = wave_sum64(w0);
+    w1 = wave_sum64(w1);
+    // columns before j hold their reflectors in the rows from j on (v_j is
+    // zero above), so w is S(c, j); columns after j are projected
+    const int c0 = 2 * wave, c1 = c0 + 1;
+    if (lane == 0 && c0 < j) S[c0][j] = w0;
+    if (lane == 0 && c1 < j) S[c1][j] = w1;
+    const double tj = tau[j];
+    const double f0 = c0 > j ? w0 * tj : 0.0, f1 = c1 > j ? w1 * tj : 0.0;
+#pragma unroll
+    for (int t = 0; t < NRL; ++t) {
+      a0[t] -= f0 * v[t];
+      a1[t] -= f1 * v[t];
+    }
+  }
+  __syncthreads();
+  // T(0:j, j) = -tau_j T(0:j, 0:j) S(0:j, j), T(j, j) = tau_j (dlarft): lane
+  // i of the last wave owns row i, the others store R and V
+  if (wave == kQrWaves - 1 && lane < kQrPanel) {
+    for (int j = 0; j < pc; ++j) {
+      // whole steps of eight: T and S are zero past the triangle
+      double e[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      for (int l = 0; l < j; l += 8)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) e[q] += T[lane][l + q] * S[l + q][j];
+      const double sum = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+      T[lane][j] = lane < j ? -tau[j] * sum : (lane == j ? tau[j] : 0.0);
+    }
+  }
+  // R (the panel's upper triangle) back in place, V explicit from here on
+  auto finish = [&](double (&a)[NRL], int c) {
+    if (c < pc) {   // uniform
+      if (lane <= c && lane < rows) X[lane + ld * c] = a[0];
+      a[0] = lane > c ? a[0] : (lane == c ? 1.0 : 0.0);
+#pragma unroll
+      for (int t = 0; t < NRL; ++t)
+        if (lane + 64 * t < rows) Vb[lane + 64 * t + (int64_t)rows * c] = a[t];
+    }
+  };
+  finish(a0, 2 * wave);
+  finish(a1, 2 * wave + 1);
+  // Y = V T^T by chunks of rows through LDS: result rows j, columns r, so
+  // that consecutive lanes store consecutive rows of Y
+  constexpr int LDP = kQrChunk + 1;
+#pragma unroll
+  for (int t0 = 0; t0 < NRL; t0 += kQrChunk / 64) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kQrChunk / 64; ++t) {   // NRL is a multiple of kQrChunk / 64
+      P[2 * wave * LDP + lane + 64 * t] = a0[t0 + t];
+      P[(2 * wave + 1) * LDP + lane + 64 * t] = a1[t0 + t];
+    }
+    __syncthreads();
+    const int lr = 16 * wave + (lane & 15), r = 64 * t0 + lr;
+    if (64 * t0 + 16 * wave < rows) {   // uniform
+#pragma unroll
+      for (int tile = 0; tile < 2; ++tile) {
+        d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k0 = 0; k0 < kQrPanel; k0 += 4) {
+          const int k = k0 + (lane >> 4);
+          acc = mfma16(T[16 * tile + (lane & 15)][k], P[k * LDP + lr], acc);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int j = 16 * tile + mfma_row<double>(lane, q);
+          if (j < pc && r < rows) Yb[r + (int64_t)rows * j] = acc[q];
+        }
+      }
+    }
+  }
+}
+
+constexpr int kQrRegRows = 1024;
+// Columns per Householder panel of a p-row matrix: what the register panel
+// holds, or what fits the LDS budget of longer ones.
+int qr_panel_columns(int p) { return p <= kQrRegRows ? kQrPanel : std::min(kQrPanel, kSvdLdsDoubles / (p | 1)); }
+
+// Factorises the panel X (rows x pc) of each of nb matrices.
+void qr_panel(int rows, int pc, double* X, int64_t ld, double* Vb, double* Yb, int nb, int64_t sX, int64_t sVY,
+              hipStream_t st) {
+  const dim3 grid(1, (unsigned)nb);
+  if (rows <= kQrRegRows) {
+    constexpr int kP = kQrPanel * (kQrChunk + 1);
+    static std::atomic<bool> attr_set{false};   // concurrent first calls only repeat the call
+    if (!attr_set) {
+      for (auto f : {qr_panel_reg_kernel<4>, qr_panel_reg_kernel<8>, qr_panel_reg_kernel<12>, qr_panel_reg_kernel<16>})
+        TTF_HIP(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)(sizeof(double) * kP)));
+      attr_set = true;
+    }
+    auto kern = rows <= 256 ? qr_panel_reg_kernel<4> : rows <= 512 ? qr_panel_reg_kernel<8>
+              : rows <= 768 ? qr_panel_reg_kernel<12> : qr_panel_reg_kernel<16>;
+    static_assert(kP >= 2 * kQrRegRows, "the reflector buffers share the staging area");
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kQrWaves), sizeof(double) * kP, st, rows, pc, X, ld, Vb, Yb, sX, sVY);
+  } else {
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set) {
+      TTF_HIP(hipFuncSetAttribute((const void*)qr_panel_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(sizeof(double) * kSvdLdsDoubles)));
+      attr_set = true;
+    }
+    hipLaunchKernelGGL(qr_panel_kernel, grid, dim3(256), sizeof(double) * (size_t)pc * (rows | 1), st, rows, pc, X, ld,
+                       Vb, Yb, sX, sVY);
+  }
+  TTF_HIP(hipGetLastError());
+}
+
 // X (q x q, ld q) = P R^T for the upper triangle R of W (ld ldw): row i of
 // R^T goes to row rowperm[i] of X.
 __global__ void upper_transpose_kernel(int q, const double* __restrict__ W, int64_t ldw,
@@ -1045,27 +1240,16 @@ int sorted_norms(int mw, int k, const double* X, double small2, std::vector<doub
 // columns (as many as fit the LDS budget with p rows) in one launch for the
 // whole batch, trailing columns updated by two batched GEMMs.
 void qr_r_factor_batched(int p, int q, double* W, int nb, int64_t sW, hipStream_t st) {
-  const int lp = p | 1;
-  const int pcmax = std::min(kQrPanel, kSvdLdsDoubles / lp);
+  const int pcmax = qr_panel_columns(p);
   TTF_REQUIRE(pcmax >= 1, "qr: %d rows exceed the panel LDS budget", p);
   TTF_REQUIRE(nb >= 1 && nb <= 65535, "qr: batch of %d", nb);
-  static std::atomic<bool> attr_set{false};   // concurrent first calls only repeat the call
-  if (!attr_set) {
-    TTF_HIP(hipFuncSetAttribute((const void*)qr_panel_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * kSvdLdsDoubles)));
-    attr_set = true;
-  }
   const int64_t sVY = (int64_t)p * kQrPanel, sZ = (int64_t)kQrPanel * q;
   double* Vb = (double*)arena(kArenaTrunc3, sizeof(double) * (size_t)nb * (2 * sVY + sZ));
   double* Yb = Vb + (size_t)nb * sVY;
   double* Z = Yb + (size_t)nb * sVY;
   for (int k0 = 0; k0 < q; k0 += pcmax) {
     const int rows = p - k0, pc = std::min(pcmax, q - k0);
-    const size_t lds = sizeof(double) * (size_t)pc * (rows | 1);
-    double* Xp = W + k0 + (int64_t)p * k0;
-    hipLaunchKernelGGL(qr_panel_kernel, dim3(1, nb), dim3(256), lds, st, rows, pc, Xp, (int64_t)p, Vb, Yb, sW,
-                       sVY);
-    TTF_HIP(hipGetLastError());
+    qr_panel(rows, pc, W + k0 + (int64_t)p * k0, p, Vb, Yb, nb, sW, sVY, st);
     const int nrest = q - k0 - pc;
     if (nrest > 0) {
       double* Cm = W + k0 + (int64_t)p * (k0 + pc);
@@ -1126,7 +1310,7 @@ __global__ void tsqr_copy_r_kernel(int q, const double* __restrict__ S, int64_t 
 // the R obtained differs from the direct one only by the signs of its rows.
 void qr_r_factor(int p, int q, double* W, hipStream_t st) {
   const int h = std::max(q, std::min(4 * q, 256));
-  const int pc_direct = std::max(1, std::min(kQrPanel, kSvdLdsDoubles / (p | 1)));
+  const int pc_direct = std::max(1, qr_panel_columns(p));
   if (q > 128 || p <= 2 * h || ceil_div(q, pc_direct) <= 4) {
     qr_r_factor_batched(p, q, W, 1, 0, st);
     return;
@@ -1256,15 +1440,8 @@ __global__ void upper_copy_kernel(int k, int m, const double* __restrict__ W, in
 void householder_qr(int n, int m, const double* A, double* Q, double* R, int64_t ldr, hipStream_t st) {
   TTF_REQUIRE(n >= 1 && m >= 1, "householder_qr: invalid sizes %d x %d", n, m);
   const int k = std::min(n, m);
-  const int lp = n | 1;
-  const int pcmax = std::min(kQrPanel, kSvdLdsDoubles / lp);
+  const int pcmax = qr_panel_columns(n);
   TTF_REQUIRE(pcmax >= 1, "householder_qr: %d rows exceed the panel LDS budget", n);
-  static std::atomic<bool> attr_set{false};
-  if (!attr_set) {
-    TTF_HIP(hipFuncSetAttribute((const void*)qr_panel_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * kSvdLdsDoubles)));
-    attr_set = true;
-  }
   // workspace: W (n x m) | every panel's V and Y (rows x pc each, <= n x k) | Z (pc x max(m, k))
   const size_t vy = (size_t)n * k;
   double* W = (double*)arena(kArenaTrunc2, sizeof(double) * ((size_t)n * m + 2 * vy + (size_t)kQrPanel * std::max(m, k)));
@@ -1280,10 +1457,7 @@ void householder_qr(int n, int m, const double* A, double* Q, double* R, int64_t
     double* Yb = Yall + used;
     off.push_back(used);
     used += (int64_t)rows * pc;
-    const size_t lds = sizeof(double) * (size_t)pc * (rows | 1);
-    hipLaunchKernelGGL(qr_panel_kernel, dim3(1, 1), dim3(256), lds, st, rows, pc, W + k0 + (int64_t)n * k0,
-                       (int64_t)n, Vb, Yb, (int64_t)0, (int64_t)0);
-    TTF_HIP(hipGetLastError());
+    qr_panel(rows, pc, W + k0 + (int64_t)n * k0, n, Vb, Yb, 1, 0, 0, st);
     const int nrest = m - k0 - pc;
     if (nrest > 0) {
       // trailing columns: C <- H^T C = C - Y (V^T C)
