@@ -149,7 +149,10 @@ __device__ void write_sorted(double (*A)[LD], double (*V)[LD], int n, int desc, 
   }
 }
 
-__global__ __launch_bounds__(256) void syev_small_kernel(int n, double* Aall, double* wall,
+// A thread per 2x2 block of the Jacobi rounds: 256 threads up to order 32,
+// 1024 past it (up to 1068 us at orders 33 to 64 with 256 threads and four
+// blocks each, up to 603 us with 1024).
+__global__ __launch_bounds__(1024) void syev_small_kernel(int n, double* Aall, double* wall,
                                                          double* Qall, int desc) {
   __shared__ double A[64][65], B[64][65];
   __shared__ double V[64][65];
@@ -172,7 +175,7 @@ __global__ __launch_bounds__(256) void syev_small_kernel(int n, double* Aall, do
 void syev_small(int n, int count, double* A, double* w, double* Q, int desc, hipStream_t st) {
   TTF_REQUIRE(n >= 1 && n <= 64, "syev_small: n=%d out of range (1..64)", n);
   if (count <= 0) return;
-  hipLaunchKernelGGL(syev_small_kernel, dim3(count), dim3(256), 0, st, n, A, w, Q, desc);
+  hipLaunchKernelGGL(syev_small_kernel, dim3(count), dim3(n <= 32 ? 256 : 1024), 0, st, n, A, w, Q, desc);
   TTF_HIP(hipGetLastError());
 }
 
@@ -985,63 +988,99 @@ void complete_columns(int m, int k0, int k, double* U, int64_t ldu, hipStream_t 
 }
 
 // ---- Cholesky QR of nearly orthonormal columns
-// G (q x q, ld q) = R^T R by right-looking Cholesky in LDS and the inverse of
-// the upper factor: Rinv (q x q, ld q, upper).  LDS holds R in the upper
-// triangle of a (q+1) x (q+1) array and column j of R^-1 in its row j+1 (the
-// strictly lower part), so both fit at once.  *info = k+1 when the k-th
-// pivot is not positive.  One work-group, q <= kCholMax.
+// G (q x q, ld q) = R^T R and the inverse of the upper factor: Rinv (q x q,
+// ld q, upper).  *info = k+1 when the k-th pivot is not positive.  One
+// work-group of 256, q <= 16 TS, the symmetrised G in registers: thread t owns
+// the TS x TS tile at rows TS (t % 16) and columns TS (t / 16), padded with the
+// identity.  With G = L D L^T, step k subtracts f_i = a_ik / a_kk times row k
+// from the rows below it and leaves -f_i in column k, so that row i ends as
+// the unscaled row of L^-1 in its first i entries (the elimination of [G I]
+// in place) and R^-1 = L^-T D^-1/2.  Column k and row k go through LDS,
+// double-buffered: one barrier a step.  Order 96: 434 us with the factor in
+// LDS and a back substitution per thread -> 91 us; order 64 now 21 us.
 constexpr int kCholMax = 128;
 
+template <int TS>
 __global__ __launch_bounds__(256) void chol_inv_kernel(int q, const double* __restrict__ G,
                                                        double* __restrict__ Rinv, int* __restrict__ info) {
-  extern __shared__ double L[];
-  __shared__ int fail;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int ld = q + 1;
-  for (int e = tid; e < q * q; e += nt) {
-    const int i = e % q, j = e / q;
-    if (i <= j) L[i * ld + j] = 0.5 * (G[i + (int64_t)q * j] + G[j + (int64_t)q * i]);
-  }
-  if (tid == 0) fail = 0;
-  for (int k = 0; k < q; ++k) {
-    __syncthreads();
-    if (tid == 0) {
-      const double d = L[k * ld + k];
-      if (d > 0.0) L[k * ld + k] = sqrt(d);
-      else fail = k + 1;
+  __shared__ double colb[2][16 * TS], rowb[2][16 * TS], piv[16 * TS];
+  const int t = threadIdx.x, ti = t & 15, tj = t >> 4;
+  double a[TS][TS];
+#pragma unroll
+  for (int s = 0; s < TS; ++s)
+#pragma unroll
+    for (int r = 0; r < TS; ++r) {
+      const int i = min(TS * ti + r, q - 1), j = min(TS * tj + s, q - 1);
+      a[r][s] = 0.5 * (G[i + (int64_t)q * j] + G[j + (int64_t)q * i]);
     }
-    __syncthreads();
-    if (fail) break;
-    const double rkk = L[k * ld + k];
-    for (int j = k + 1 + tid; j < q; j += nt) L[k * ld + j] /= rkk;
-    __syncthreads();
-    const int w = q - k - 1;
-    for (int e = tid; e < w * w; e += nt) {
-      const int i = k + 1 + e % w, j = k + 1 + e / w;
-      if (i <= j) L[i * ld + j] -= L[k * ld + i] * L[k * ld + j];
+#pragma unroll
+  for (int s = 0; s < TS; ++s)
+#pragma unroll
+    for (int r = 0; r < TS; ++r) {
+      const int i = TS * ti + r, j = TS * tj + s;
+      a[r][s] = (i < q && j < q) ? a[r][s] : (i == j ? 1.0 : 0.0);
+    }
+  int bad = 0;
+  for (int kb = 0; kb < (q + TS - 1) / TS; ++kb) {
+    const bool rowk = ti == kb, colk = tj == kb, below = ti > kb;
+#pragma unroll
+    for (int c = 0; c < TS; ++c) {
+      const int k = TS * kb + c;
+      if (k < q) {   // uniform
+        const int buf = k & 1;
+        if (colk) {
+#pragma unroll
+          for (int r = 0; r < TS; ++r) colb[buf][TS * ti + r] = a[r][c];
+        }
+        if (rowk) {
+#pragma unroll
+          for (int s = 0; s < TS; ++s) rowb[buf][TS * tj + s] = a[c][s];
+        }
+        __syncthreads();
+        const double pv = rowb[buf][k];
+        bad = (bad == 0 && !(pv > 0.0)) ? k + 1 : bad;
+        if (t == 0) piv[k] = pv;
+        const double inv = 1.0 / pv;
+        double f[TS], h[TS];
+#pragma unroll
+        for (int r = 0; r < TS; ++r) f[r] = colb[buf][TS * ti + r] * inv;
+#pragma unroll
+        for (int s = 0; s < TS; ++s) h[s] = rowb[buf][TS * tj + s];
+#pragma unroll
+        for (int r = 0; r < TS; ++r) {
+          const bool down = below || (rowk && r > c);
+#pragma unroll
+          for (int s = 0; s < TS; ++s) {
+            const double v = (s == c && colk) ? -f[r] : a[r][s] - f[r] * h[s];
+            a[r][s] = down ? v : a[r][s];
+          }
+        }
+      }
     }
   }
   __syncthreads();
-  if (fail) {
-    if (tid == 0) *info = fail;
+  if (bad) {   // every thread read the same pivots
+    if (t == 0) *info = bad;
     return;
   }
-  // column j of X = R^-1 by back substitution, kept in row j+1 of L
-  for (int j = tid; j < q; j += nt) {
-    double* x = L + (j + 1) * ld;
-    x[j] = 1.0 / L[j * ld + j];
-    for (int i = j - 1; i >= 0; --i) {
-      double acc = 0.0;
-      for (int l = i + 1; l <= j; ++l) acc += L[i * ld + l] * x[l];
-      x[i] = -acc / L[i * ld + i];
+  // Rinv(j, i) = L^-1(i, j) / sqrt(d_i) for j <= i (unit diagonal), zero below
+#pragma unroll
+  for (int r = 0; r < TS; ++r) {
+    const int i = TS * ti + r;
+    const double d = i < q ? 1.0 / sqrt(piv[i]) : 0.0;
+#pragma unroll
+    for (int s = 0; s < TS; ++s) {
+      const int j = TS * tj + s;
+      if (i < q && j < q) Rinv[j + (int64_t)q * i] = j < i ? a[r][s] * d : (j == i ? d : 0.0);
     }
   }
-  __syncthreads();
-  for (int e = tid; e < q * q; e += nt) {
-    const int i = e % q, j = e / q;
-    Rinv[e] = (i <= j) ? L[(j + 1) * ld + i] : 0.0;
-  }
-  if (tid == 0) *info = 0;
+  if (t == 0) *info = 0;
+}
+
+void chol_inv(int q, const double* G, double* Rinv, int* info, hipStream_t st) {
+  auto kern = q <= 32 ? chol_inv_kernel<2> : q <= 64 ? chol_inv_kernel<4> : chol_inv_kernel<8>;
+  hipLaunchKernelGGL(kern, dim3(1), dim3(256), 0, st, q, G, Rinv, info);
+  TTF_HIP(hipGetLastError());
 }
 
 __global__ void scale_cols_kernel(int m, int k, double* __restrict__ U, int64_t ldu, const double* __restrict__ sc) {
@@ -1058,22 +1097,14 @@ __global__ void scale_cols_kernel(int m, int k, double* __restrict__ U, int64_t 
 bool cholqr2(int p, int k, double* U, int64_t ldu, hipStream_t st) {
   if (k <= 0) return true;
   TTF_REQUIRE(k <= kCholMax, "cholqr2: %d columns exceed %d", k, kCholMax);
-  static std::atomic<bool> attr_set{false};   // concurrent first calls only repeat the call
-  if (!attr_set) {
-    TTF_HIP(hipFuncSetAttribute((const void*)chol_inv_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * (kCholMax + 1) * (kCholMax + 1))));
-    attr_set = true;
-  }
   double* G = (double*)arena(kArenaSvdLong, sizeof(double) * ((size_t)2 * k * k + (size_t)p * k) + 64);
   double* Ri = G + (size_t)k * k;
   double* T = Ri + (size_t)k * k;
   int* info = (int*)(T + (size_t)p * k);
-  const size_t lds = sizeof(double) * (size_t)(k + 1) * (k + 1);
   for (int pass = 0; pass < 2; ++pass) {
     if (k <= 64) tsgram(p, k, k, U, ldu, U, ldu, G, k, st);
     else gemm_launch(colmajor<double>('T', 'N', k, k, p, 1.0, U, ldu, U, ldu, 0.0, G, k), st);
-    hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(256), lds, st, k, G, Ri, info);
-    TTF_HIP(hipGetLastError());
+    chol_inv(k, G, Ri, info, st);
     int hinfo = 0;
     read_back(&hinfo, info, sizeof(int), st);
     if (hinfo != 0) return false;
