@@ -149,8 +149,9 @@ __device__ void write_sorted(double (*A)[LD], double (*V)[LD], int n, int desc, 
   }
 }
 
-// A thread per 2x2 block of the Jacobi rounds: 256 threads up to order 32,
-// 1024 past it (up to 1068 us at orders 33 to 64 with 256 threads and four
+// A thread per 2x2 block of the Jacobi rounds, and up to order 32 as many
+// again for the rotations and the vectors: 512 threads up to there, 1024 past
+// it (up to 1068 us at orders 33 to 64 with 256 threads and four
 // blocks each, up to 603 us with 1024).
 __global__ __launch_bounds__(1024) void syev_small_kernel(int n, double* Aall, double* wall,
                                                          double* Qall, int desc) {
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(1024) void syev_small_kernel(int n, double* Aall, d
 void syev_small(int n, int count, double* A, double* w, double* Q, int desc, hipStream_t st) {
   TTF_REQUIRE(n >= 1 && n <= 64, "syev_small: n=%d out of range (1..64)", n);
   if (count <= 0) return;
-  hipLaunchKernelGGL(syev_small_kernel, dim3(count), dim3(n <= 32 ? 256 : 1024), 0, st, n, A, w, Q, desc);
+  hipLaunchKernelGGL(syev_small_kernel, dim3(count), dim3(n <= 32 ? 512 : 1024), 0, st, n, A, w, Q, desc);
   TTF_HIP(hipGetLastError());
 }
 
@@ -193,6 +194,8 @@ void syev_small(int n, int count, double* A, double* w, double* Q, int desc, hip
 //      largest coupling measured here (the same quantity that decides a
 //      rotation) drives the sweep loop, so a sweep without rotations ends it;
 //   3. P back to X and, with V, V(:, pair) <- V(:, pair) Qp by MFMA.
+// Without V and with one sweep a pair (the default), svd_pair_gram_kernel
+// takes the rotations of step 2 from G itself.
 // Columns whose squared norm is below the rounding floor small2 are treated
 // as zero and never rotated.
 constexpr int kSvdMaxP = 32;          // columns per pair (2b) at most
@@ -553,6 +556,151 @@ __global__ __launch_bounds__(16 * LPP) void svd_pair_kernel(int mw, int nw, int 
   lds_apply_rotation(lds, nw, ldv, n, Qc);
   __syncthreads();
   lds_to_cols(lds, ldv, nw, n, V, nw, cols);
+}
+
+// G (n x n, n <= 32, row stride LDG) = P^T P for the LDS columns P (rows x n,
+// column stride ld) times `scale` on eight waves: four 16x16 tiles, the rows
+// split in two.  `scratch` holds 1024 doubles.  Ends with a block barrier.
+template <int LDG>
+__device__ inline void lds_gram8(const double* P, int rows, int ld, int n, double scale, double (*G)[LDG],
+                                 double* scratch) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int tile = wv & 3, part = wv >> 2, ti = tile >> 1, tj = tile & 1;
+  const int per = ((rows + 1) / 2 + 3) / 4 * 4;
+  const int kbeg = part * per, kend = min(rows, kbeg + per);
+  const int ci = ti * 16 + (lane & 15), cj = tj * 16 + (lane & 15), kk = lane >> 4;
+  const bool va = ci < n, vb = cj < n;
+  const double* pa = P + (va ? ci : 0) * ld;
+  const double* pb = P + (vb ? cj : 0) * ld;
+  d4_t acc[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) acc[u] = d4_t{0.0, 0.0, 0.0, 0.0};
+  if (16 * ti < n && 16 * tj < n) {   // uniform
+    for (int k0 = kbeg; k0 < kend; k0 += 64) {
+      // 64 rows a step; lane group kk takes rows k0 + 16 kk + u, so that with
+      // the odd stride a wave's 64 loads touch every bank the same number of
+      // times.  Rows past the end and columns past n read valid ones and are
+      // zeroed.
+#pragma unroll
+      for (int u0 = 0; u0 < 16; u0 += 8) {
+        double a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = min(k0 + 16 * kk + u0 + u, kend - 1);
+          a[u] = pa[r];
+          b[u] = pb[r];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const bool in = k0 + 16 * kk + u0 + u < kend;
+          acc[u & 3] = mfma16(in && va ? a[u] : 0.0, in && vb ? b[u] : 0.0, acc[u & 3]);
+        }
+      }
+    }
+  }
+  const d4_t sum = (acc[0] + acc[2]) + (acc[1] + acc[3]);
+  if (part == 1)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) scratch[256 * tile + 64 * r + lane] = sum[r];
+  __syncthreads();
+  if (part == 0)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      G[ti * 16 + mfma_row<double>(lane, r)][cj] = (sum[r] + scratch[256 * tile + 64 * r + lane]) * scale;
+  __syncthreads();
+}
+
+// The pair step of the preconditioned Jacobi (columns of P R^T, no V) with
+// the rotations taken from the pair's Gram matrix: one sweep of two-sided
+// rotations on the 32 x 32 Gram in slot order (jacobi.h), their product
+// accumulated beside it, and one matrix-core product that applies it to the
+// columns.  A round then costs a 2x2 block per thread in place of dot
+// products over the rows; the Gram drifts from the columns' own inside a
+// launch, but every launch forms it afresh, and that fresh Gram decides the
+// rotations' relative tolerance, the skip and the convergence, as the
+// column form's dot products do.  `scale` (a power of two near 1 / ||W||_F^2)
+// keeps the squares of the Gram's entries in range, with small2 scaled alike.
+// 256 rows, 32 columns: 40.2 us with the column form -> 27.8 us; the number
+// of sweeps is unchanged.  Bound by the chain of the 31 rounds (37800 of
+// 62000 clocks; the Gram 9000, the update 7900, the loads 6000).
+constexpr int kPairLd = 34;   // row stride of the 32 x 32 work matrices (jacobi.h: even)
+
+__global__ __launch_bounds__(512) void svd_pair_gram_kernel(int mw, int nw, int bsz, int nb, int round,
+                                                            double* __restrict__ W, double scale, double small2,
+                                                            double tol, unsigned long long* offmax) {
+  extern __shared__ double lds[];   // pair columns: column j at lds + j * ldp
+  __shared__ double A[kSvdMaxP + 1][kPairLd], B[kSvdMaxP + 1][kPairLd], V[kSvdMaxP + 1][kPairLd];
+  __shared__ double dinv[kSvdMaxP];
+  __shared__ int cols[kSvdMaxP];
+  __shared__ int flags[3];
+  __shared__ unsigned long long cmax;
+  const int tid = threadIdx.x;
+  int bi, bj;
+  circle_pair(round, blockIdx.x, nb, &bi, &bj);
+  const int nf = max(0, min(bsz, nw - bi * bsz)), n = nf + max(0, min(bsz, nw - bj * bsz));
+  if (n == 0 || nf == 0 || nf == n) return;   // a block beyond the last column
+  if (tid < n) cols[tid] = tid < nf ? bi * bsz + tid : bj * bsz + tid - nf;
+  if (tid == 0) cmax = 0ull;
+  __syncthreads();
+  const int ldp = mw | 1;                     // odd stride: conflict-free fragment loads
+  cols_to_lds(W, mw, cols, mw, n, lds, ldp);
+  __syncthreads();
+  lds_gram8<kPairLd>(lds, mw, ldp, n, scale, A, &V[0][0]);
+  if (tid < n) dinv[tid] = A[tid][tid] > small2 ? 1.0 / sqrt(A[tid][tid]) : 0.0;
+  __syncthreads();
+  {
+    double cm = 0.0;
+    for (int e = tid; e < kSvdMaxP * kSvdMaxP; e += blockDim.x) {
+      const int i = e % kSvdMaxP, j = e / kSvdMaxP;   // kSvdMaxP is a power of two
+      if (i < j && j < n) cm = fmax(cm, fabs(A[i][j]) * dinv[i] * dinv[j]);
+      V[i][j] = i == j ? 1.0 : 0.0;
+    }
+    block_max_into(cm, &cmax);
+  }
+  __syncthreads();
+  if (__longlong_as_double((long long)cmax) <= 0.5 * tol) return;
+  if (tid == 0) atomicMax(offmax, cmax);
+  const double tol2 = tol * tol;
+  jacobi_sym_slots<kPairLd>(
+      A, B, V, n, 1,
+      [=](double gpq, double gpp, double gqq) {
+        return gpp > small2 && gqq > small2 && gpq * gpq > tol2 * (gpp * gqq);
+      },
+      flags, 0.0);
+  if (flags[0] == 0) return;   // no rotation
+  // W's columns <- (LDS columns) V, 16 rows a wave: the product's transpose,
+  // so that 16 lanes store 16 consecutive rows of a column
+  const int lane = tid & 63, l16 = lane & 15, kk = lane >> 4;
+  double q[2][kSvdMaxP / 4];
+#pragma unroll
+  for (int t = 0; t < kSvdMaxP / 4; ++t) {
+    const int k = 4 * t + kk;
+    q[0][t] = V[k][l16];
+    q[1][t] = V[k][16 + l16];
+  }
+  for (int r0 = (tid >> 6) * 16; r0 < mw; r0 += 128) {
+    const int row = r0 + l16;
+    const double* x = lds + min(row, mw - 1);
+    double b[kSvdMaxP / 4];
+#pragma unroll
+    for (int t = 0; t < kSvdMaxP / 4; ++t) b[t] = x[min(4 * t + kk, n - 1) * ldp];
+#pragma unroll
+    for (int t = 0; t < kSvdMaxP / 4; ++t) b[t] = 4 * t + kk < n ? b[t] : 0.0;
+    d4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+    for (int t = 0; t < kSvdMaxP / 4; ++t) {
+      acc[0] = mfma16(q[0][t], b[t], acc[0]);
+      acc[1] = mfma16(q[1][t], b[t], acc[1]);
+    }
+    if (row < mw)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * h + mfma_row<double>(lane, r);
+          if (j < n) W[(int64_t)cols[j] * mw + row] = acc[h][r];
+        }
+  }
 }
 
 // ---- Householder QR (R factor only) for the preconditioning of the Jacobi
@@ -1217,6 +1365,16 @@ JacobiResult jacobi_columns(int mw, int nw, double* X, double* V, hipStream_t st
     attr_set = true;
   }
   const int inner = svd_inner_sweeps();
+  const bool gram = V == nullptr && inner == 1;
+  const double scale = std::ldexp(1.0, -std::min(std::max(std::ilogb(fro2), -1000), 1000));
+  if (gram) {
+    static std::atomic<bool> gattr{false};
+    if (!gattr) {
+      TTF_HIP(hipFuncSetAttribute((const void*)svd_pair_gram_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(sizeof(double) * kSvdLdsDoubles)));
+      gattr = true;
+    }
+  }
   unsigned long long hoff = 0;
   // Convergence is quadratic at the end: after a sweep whose largest
   // coupling (measured before its rotations) was at most kQuadStop, the
@@ -1228,8 +1386,12 @@ JacobiResult jacobi_columns(int mw, int nw, double* X, double* V, hipStream_t st
   for (res.sweeps = 1; res.sweeps <= 60; ++res.sweeps) {
     TTF_HIP(hipMemsetAsync(offmax, 0, sizeof(unsigned long long), st));
     for (int r = 0; r < nb - 1; ++r) {
-      hipLaunchKernelGGL(kern, dim3(nb / 2), dim3(threads), lds, st, mw, nw, bsz, nb, r, X, V, res.small2, tol,
-                         inner, offmax);
+      if (gram)
+        hipLaunchKernelGGL(svd_pair_gram_kernel, dim3(nb / 2), dim3(512), lds, st, mw, nw, bsz, nb, r, X, scale,
+                           scale * res.small2, tol, offmax);
+      else
+        hipLaunchKernelGGL(kern, dim3(nb / 2), dim3(threads), lds, st, mw, nw, bsz, nb, r, X, V, res.small2, tol,
+                           inner, offmax);
       TTF_HIP(hipGetLastError());
     }
     read_back(&hoff, offmax, sizeof(hoff), st);

@@ -230,9 +230,11 @@ void orth_block(int k, const double* G, double* T, int* mask, hipStream_t st, in
 // LD: rr_kernel<33, 34> serves m <= 32 (the even stride keeps each
 // thread's pair of Jacobi block entries 16-byte aligned for one load; the
 // 24x24 Jacobi measured 12% faster than with the stride 65) and
-// rr_kernel<kMaxM, kMaxM + 1> the rest (launch_rr picks).
+// rr_kernel<kMaxM, kMaxM + 1> the rest (launch_rr picks).  512 threads leave
+// waves without 2x2 blocks for the rotations and the vectors (52 us a call at
+// m = 24 with 256 threads and two barriers a round, 46 us so).
 template <int MR, int LD>
-__global__ __launch_bounds__(256) void rr_kernel(int m, int bs, int nx, const double* __restrict__ H,
+__global__ __launch_bounds__(512) void rr_kernel(int m, int bs, int nx, const double* __restrict__ H,
                                                  const int* __restrict__ maskP_in, const int* __restrict__ maskW,
                                                  double* __restrict__ theta, double* __restrict__ CZ,
                                                  int* __restrict__ maskP, double* __restrict__ amax,
@@ -362,10 +364,10 @@ __global__ __launch_bounds__(256) void rr_kernel(int m, int bs, int nx, const do
 static void launch_rr(hipStream_t st, int m, int bs, int nx, const double* H, const int* maskP_in, const int* maskW,
                       double* theta, double* CZ, int* maskP, double* amax, int lower) {
   if (m <= 32)
-    hipLaunchKernelGGL((rr_kernel<33, 34>), dim3(1), dim3(256), 0, st, m, bs, nx, H, maskP_in, maskW, theta, CZ,
+    hipLaunchKernelGGL((rr_kernel<33, 34>), dim3(1), dim3(512), 0, st, m, bs, nx, H, maskP_in, maskW, theta, CZ,
                        maskP, amax, lower);
   else
-    hipLaunchKernelGGL((rr_kernel<kMaxM, kMaxM + 1>), dim3(1), dim3(256), 0, st, m, bs, nx, H, maskP_in, maskW,
+    hipLaunchKernelGGL((rr_kernel<kMaxM, kMaxM + 1>), dim3(1), dim3(512), 0, st, m, bs, nx, H, maskP_in, maskW,
                        theta, CZ, maskP, amax, lower);
 }
 
