@@ -151,9 +151,8 @@ __device__ void write_sorted(double (*A)[LD], double (*V)[LD], int n, int desc, 
 
 // A thread per 2x2 block of the Jacobi rounds, and up to order 32 as many
 // again for the rotations and the vectors: 512 threads up to there, 1024 past
-// it (up to 1068 us at orders 33 to 64 with 256 threads and four
-// blocks each, up to 603 us with 1024, 818 us with one
-// barrier a round).
+// it (orders 33 to 64, up to 1068 us with 256 threads and four blocks each, up
+// to 534 us with 1024).
 __global__ __launch_bounds__(1024) void syev_small_kernel(int n, double* Aall, double* wall,
                                                          double* Qall, int desc) {
   __shared__ double A[64][65], B[64][65];
