@@ -43,21 +43,3 @@ def test_orders(ttlib, n):
         assert np.abs(wi - np.linalg.eigvalsh(a)).max() <= tol * np.linalg.norm(a)
         assert np.abs(qi.T @ qi - np.eye(n)).max() <= tol
         assert np.abs(a @ qi - qi * wi).max() <= tol * np.linalg.norm(a)
-
-
-@pytest.mark.parametrize("n", [2, 4, 27, 32, 33, 64])
-@pytest.mark.parametrize("scale", [1e-153, 1e-156, 1e-158, 1e-160, 1e151])
-def test_orders_tiny(ttlib, n, scale):
-    """Entries whose squares are subnormal, or near overflow: the vectors are
-    orthonormal and diagonalise the matrix as for entries near one (the
-    scaling is a power of two, so the bars are those of test_orders)."""
-    import ttfort
-    rng = np.random.default_rng(n)
-    a = rng.standard_normal((n, n))
-    a = a + a.T
-    w, Q = ttfort.syev_small((a * scale)[None])
-    tol = 64 * n * np.finfo(float).eps
-    w, Q = w[0] / scale, Q[0]
-    assert np.abs(w - np.linalg.eigvalsh(a)).max() <= tol * np.linalg.norm(a)
-    assert np.abs(Q.T @ Q - np.eye(n)).max() <= tol
-    assert np.abs(a @ Q - Q * w).max() <= tol * np.linalg.norm(a)

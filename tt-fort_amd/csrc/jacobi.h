@@ -436,40 +436,21 @@ __device__ double (*jacobi_sym_slots_inplace(double (*A)[LD], double (*B)[LD], d
 
 // Diagonalises the symmetric n x n matrix held in A (row stride LD, n <= 64)
 // and accumulates the rotations into V (V <- V J); B is a second buffer of
-// the same shape.  tol_abs = eps ||A||.  Returns the matrix (A or B) whose
-// diagonal holds the eigenvalues, in the order of V's columns.  Orders from 3
-// with (n + 1) / 2 squared <= blockDim.x - 64 take the slot-ordered form with a
-// wave for the rotations, up to blockDim.x the one in place, larger ones the
+// the same shape.  Returns the matrix (A or B) whose diagonal holds the
+// eigenvalues, in the order of V's columns.  Orders from 3 with (n + 1) / 2 squared
+// <= blockDim.x - 64 take the slot-ordered form with a wave for the
+// rotations, up to blockDim.x the one in place, larger ones the
 // double-buffered one.
 template <int LD>
 __device__ double (*jacobi_sym(double (*A)[LD], double (*B)[LD], double (*V)[LD], int n, int max_sweeps,
                                double tol_abs, int* flags, double small = kJacobiSmall))[LD] {
-  // The rotations form squares of differences and couplings, down to that of
-  // tol_abs = eps ||A||.  Where those would leave the normal range (c^2 + s^2
-  // would then miss 1 by their rounding: 1e-8 for entries near 1e-158) the
-  // matrix is scaled by a power of two first and its diagonal back at the end.
-  const int ex = tol_abs > 0.0 ? __builtin_amdgcn_frexp_exp(tol_abs) + 52 : 0;   // of ||A||
-  const bool scaled = n >= 2 && (ex < -450 || ex > 500);   // uniform
-  if (scaled) {
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) A[e % n][e / n] = ldexp(A[e % n][e / n], -ex);
-    tol_abs = ldexp(tol_abs, -ex);
-    __syncthreads();
-  }
   const auto go = [tol_abs](double apq, double app, double aqq) { return jacobi_go(apq, app, aqq, tol_abs); };
   const int half = (n + 1) / 2;
-  double(*D)[LD];
   if (n >= 3 && half * half <= (int)blockDim.x - 64)
-    D = jacobi_sym_slots<LD>(A, B, V, n, max_sweeps, go, flags, small);
-  else if (n >= 2 && half * half <= (int)blockDim.x)
-    D = jacobi_sym_slots_inplace<LD>(A, B, V, n, max_sweeps, go, flags, small);
-  else
-    D = jacobi_sym_circle<LD>(A, B, V, n, max_sweeps, go, flags, small);
-  if (scaled) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) D[i][i] = ldexp(D[i][i], ex);
-    __syncthreads();
-  }
-  return D;
+    return jacobi_sym_slots<LD>(A, B, V, n, max_sweeps, go, flags, small);
+  if (n >= 2 && half * half <= (int)blockDim.x)
+    return jacobi_sym_slots_inplace<LD>(A, B, V, n, max_sweeps, go, flags, small);
+  return jacobi_sym_circle<LD>(A, B, V, n, max_sweeps, go, flags, small);
 }
 
 // Block-wide sum of v over all threads (blockDim.x a multiple of 64, at most
