@@ -43,3 +43,28 @@ def test_orders(ttlib, n):
         assert np.abs(wi - np.linalg.eigvalsh(a)).max() <= tol * np.linalg.norm(a)
         assert np.abs(qi.T @ qi - np.eye(n)).max() <= tol
         assert np.abs(a @ qi - qi * wi).max() <= tol * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("n", [60, 64])
+def test_rotations_orthogonal(ttlib, n):
+    """Ten sweeps give every column 10 (n - 1) rotations, each of which may
+    miss c^2 + s^2 = 1 by its rounding, eps: at random signs
+    ||Q^T Q - I||_F = sqrt(n * 10 (n - 1)) eps, over 32 matrices on average."""
+    import ttfort
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((32, n, n))
+    _, Q = ttfort.syev_small(A + A.transpose(0, 2, 1))
+    miss = np.mean([np.linalg.norm(q.T @ q - np.eye(n)) for q in Q])
+    assert miss <= np.sqrt(10.0 * n * (n - 1)) * np.finfo(float).eps
+
+
+@pytest.mark.parametrize("n", [4, 27, 32, 33, 64])
+@pytest.mark.parametrize("scale", [1e-153, 1e-156, 1e-158])
+def test_rotations_of_tiny_entries(ttlib, n, scale):
+    """Entries whose squares are subnormal: the rotations' angles lose digits
+    with d^2 + 4 a^2, their orthogonality does not."""
+    import ttfort
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n))
+    _, Q = ttfort.syev_small(((a + a.T) * scale)[None])
+    assert np.abs(Q[0].T @ Q[0] - np.eye(n)).max() <= 64 * n * np.finfo(float).eps
