@@ -187,16 +187,16 @@ def dominant_kernel_roofline(lib, shape, nvec, iters=50):
              x=ttfort.DeviceArray.from_numpy(rng.standard_normal(nx * nvec)),
              y=ttfort.DeviceArray((ny * nvec,)))
     ms = ctypes.c_float()
-    fused = ctypes.c_int()
     for it in (5, iters):
         ttfort.check(lib.ttf_dbfun3_chain_profile(*shape, nvec, d["phi1"].ptr, d["A"].ptr, d["phi2"].ptr,
                                                   d["x"].ptr, nx, d["y"].ptr, ny, it, ctypes.byref(ms),
-                                                  ctypes.byref(fused)), lib)
+                                                  None), lib)
     flops = sum(bfun3_stage_flops(*shape)) * nvec
     achieved = flops / (ms.value * 1e-3) / 1e12
     alg_bytes = 8 * (ry1 * rx1 * ra1 + rx2 * ra2 * ry2 + ra1 * n * m * ra2 + nvec * (nx + ny))
     traffic = measured_traffic() if (shape, nvec) == (C2_LOCAL_SHAPE, C2_BLOCK) else None
-    name = ("bfun3_fused_kernel<3> + zero fill of y" if fused.value else "bfun3 GEMM chain (three stages)")
+    name = {"fused": "bfun3_fused_kernel<3> + zero fill of y", "small": "bfun3_small_kernel",
+            "chain": "bfun3 GEMM chain (three stages)"}[ttfort.bfun3_route(shape, nvec)]
     return dict(bound="mfma", achieved=round(achieved, 3), peak=MI355X_PEAK_F64_TFLOPS,
                 unit="TFLOP/s", frac=round(achieved / MI355X_PEAK_F64_TFLOPS, 4), traffic=traffic,
                 kernel="%s: y = Phi1 A Phi2 x at (r,n,r,R)=(%d,%d,%d,%d), block %d, %.1f MFLOP per call"

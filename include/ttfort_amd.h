@@ -135,12 +135,19 @@ int ttf_dbfun3_profile(int rx1, int m, int rx2, int ry1, int n, int ry2, int ra1
                        int nvec, const double* phi1, const double* A, const double* phi2,
                        const double* x, int64_t ldx, double* y, int64_t ldy, int iters,
                        float* stage_ms);
-/* Times the whole FP64 dbfun3 as the library runs it (the fused one-launch
- * kernel and its zero fill where the shape fits, else the GEMM chain):
- * `iters` back-to-back calls between two events on the library stream,
- * after one call that settles any tuning; *ms receives the mean
- * milliseconds per call and *fused (optional) 1 if the fused kernel ran.
- * Synchronous; y is overwritten. */
+/* The way in which ttf_dbfun3 (type 'd'), ttf_sbfun3 ('s'), ttf_zbfun3 ('z')
+ * or ttf_cbfun3 ('c') forms a product of these sizes whose x and y do not
+ * overlap: *route = 0 the chain of three GEMMs, 1 the fused kernel on the
+ * matrix cores ('d' only), 2 the one-launch kernel on the vector units.  No
+ * launch is made. */
+int ttf_bfun3_route(char type, int rx1, int m, int rx2, int ry1, int n, int ry2, int ra1, int ra2, int nvec,
+                    int* route);
+/* Times the whole FP64 dbfun3 as the library runs it: `iters` back-to-back
+ * calls between two events on the library stream, after one call that
+ * settles any tuning; *ms receives the mean milliseconds per call and *fused
+ * (optional) 1 if one kernel formed the product, 0 if the GEMM chain did
+ * (ttf_bfun3_route tells the two one-launch kernels apart).  Synchronous; y
+ * is overwritten. */
 int ttf_dbfun3_chain_profile(int rx1, int m, int rx2, int ry1, int n, int ry2, int ra1, int ra2, int nvec,
                              const double* phi1, const double* A, const double* phi2, const double* x,
                              int64_t ldx, double* y, int64_t ldy, int iters, float* ms, int* fused);

@@ -231,15 +231,21 @@ void launch(const SmallArgs<T>& a, int N, unsigned grid, size_t lds, hipStream_t
 }  // namespace
 
 template <typename T>
-bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
-                 int64_t ldy, hipStream_t st) {
+bool bfun3_small_fits(const Shape& s, int nvec) {
   if (!small_enabled() || nvec < 1 || s.ra2 > kMaxCols || s.n > kMaxCols) return false;
   const int64_t R1 = (int64_t)s.rx1 * s.m, K3 = (int64_t)s.rx1 * s.ra1;
   if (R1 > 2048 || K3 > 4096 || s.ry1 > 2048) return false;
   const int A2 = bucket(s.ra2), N = bucket(s.n);
-  if (!faster_small<T>(s, nvec, A2, N)) return false;
+  return faster_small<T>(s, nvec, A2, N) && lds_need<T>(s, A2, N) <= kLdsBytes &&
+         (int64_t)s.ry2 * nvec <= 0x7fffffff / kNT;
+}
+
+template <typename T>
+bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
+                 int64_t ldy, hipStream_t st) {
+  if (!bfun3_small_fits<T>(s, nvec)) return false;
+  const int A2 = bucket(s.ra2), N = bucket(s.n);
   const size_t lds = lds_need<T>(s, A2, N);
-  if (lds > kLdsBytes || (int64_t)s.ry2 * nvec > 0x7fffffff / kNT) return false;
   SmallArgs<T> a{s.rx1, s.m, s.rx2, s.ry1, s.n, s.ry2, s.ra1, s.ra2, phi1, A, phi2, x, ldx, y, ldy};
   const unsigned grid = (unsigned)(s.ry2 * nvec);
   switch (A2) {
@@ -252,6 +258,10 @@ bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* p
   return true;
 }
 
+template bool bfun3_small_fits<double>(const Shape&, int);
+template bool bfun3_small_fits<float>(const Shape&, int);
+template bool bfun3_small_fits<hipDoubleComplex>(const Shape&, int);
+template bool bfun3_small_fits<hipFloatComplex>(const Shape&, int);
 template bool bfun3_small<double>(const Shape&, int, const double*, const double*, const double*, const double*,
                                   int64_t, double*, int64_t, hipStream_t);
 template bool bfun3_small<float>(const Shape&, int, const float*, const float*, const float*, const float*, int64_t,

@@ -33,6 +33,8 @@ bool bfun3_fused_fits(const Shape& s, int nvec);
 // A == nullptr stands for the identity (m = n = 1, ra1 = ra2).  x and y must
 // not overlap.  T: double, float, hipDoubleComplex, hipFloatComplex.
 template <typename T>
+bool bfun3_small_fits(const Shape& s, int nvec);
+template <typename T>
 bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
                  int64_t ldy, hipStream_t st);
 

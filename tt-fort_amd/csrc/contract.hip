@@ -72,6 +72,15 @@ static bool overlaps(const Shape& s, const T* x, int64_t ldx, const T* y, int64_
   return x < ye && y < xe;
 }
 
+// Which way a product of operands that do not overlap is formed.
+enum { kRouteChain = 0, kRouteFused = 1, kRouteSmall = 2 };
+template <typename T>
+static int bfun3_route(const Shape& s, int nvec) {
+  if (bfun3_small_fits<T>(s, nvec)) return kRouteSmall;
+  if (std::is_same<T, double>::value && bfun3_fused_fits(s, nvec)) return kRouteFused;
+  return kRouteChain;
+}
+
 template <typename T>
 void bfun3_chain(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x,
                  int64_t ldx, T* y, int64_t ldy, hipStream_t st) {
@@ -583,7 +592,8 @@ int ttf_dbfun3_chain_profile(int rx1, int m, int rx2, int ry1, int n, int ry2, i
     Shape s = mkshape(rx1, m, rx2, ry1, n, ry2, ra1, ra2);
     TTF_REQUIRE(iters > 0 && nvec > 0 && ms != nullptr, "ttf_dbfun3_chain_profile: bad arguments");
     hipStream_t st = stream();
-    if (fused) *fused = bfun3_fused_fits(s, nvec) && !overlaps(s, x, ldx, (const double*)y, ldy, nvec) ? 1 : 0;
+    if (fused)
+      *fused = !overlaps(s, x, ldx, (const double*)y, ldy, nvec) && bfun3_route<double>(s, nvec) != kRouteChain ? 1 : 0;
     bfun3_chain<double>(s, nvec, phi1, A, phi2, x, ldx, y, ldy, st);   // settles any tuning
     hipEvent_t e0, e1;
     TTF_HIP(hipEventCreate(&e0));
@@ -597,6 +607,21 @@ int ttf_dbfun3_chain_profile(int rx1, int m, int rx2, int ry1, int n, int ry2, i
     *ms = t / (float)iters;
     TTF_HIP(hipEventDestroy(e0));
     TTF_HIP(hipEventDestroy(e1));
+  });
+}
+
+int ttf_bfun3_route(char type, int rx1, int m, int rx2, int ry1, int n, int ry2, int ra1, int ra2, int nvec,
+                    int* route) {
+  return guarded([&] {
+    const Shape s = mkshape(rx1, m, rx2, ry1, n, ry2, ra1, ra2);
+    TTF_REQUIRE(nvec > 0 && route != nullptr, "ttf_bfun3_route: bad arguments");
+    switch (type) {
+      case 'd': *route = bfun3_route<double>(s, nvec); break;
+      case 's': *route = bfun3_route<float>(s, nvec); break;
+      case 'z': *route = bfun3_route<hipDoubleComplex>(s, nvec); break;
+      case 'c': *route = bfun3_route<hipFloatComplex>(s, nvec); break;
+      default: TTF_REQUIRE(false, "ttf_bfun3_route: unknown type '%c'", type);
+    }
   });
 }
 

@@ -79,6 +79,7 @@ _sig("ttf_dbfun3_profile", _c_int, *(_S8 + [_c_int, _vp, _vp, _vp, _vp, _c_i64, 
                                            C.POINTER(C.c_float)]))
 _sig("ttf_dbfun3_chain_profile", _c_int, *(_S8 + [_c_int, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_int,
                                                  C.POINTER(C.c_float), C.POINTER(C.c_int)]))
+_sig("ttf_bfun3_route", _c_int, C.c_char, *(_S8 + [_c_int, C.POINTER(C.c_int)]))
 for _nm in ("ttf_dphi_left", "ttf_dphi_right", "ttf_zphi_left", "ttf_zphi_right"):
     _sig(_nm, _c_int, *(_S8 + [_vp, _vp, _vp, _vp, _vp]))
 for _nm in ("ttf_dphi2_left", "ttf_dphi2_right"):
@@ -322,6 +323,15 @@ def bfun3(shape, phi1, A, phi2, x, nvec=1, dtype=np.float64, transp=False):
         fn = lib.ttf_zbfun3_transp
     check(fn(*shape, nvec, dphi1.ptr, dA.ptr, dphi2.ptr, dx.ptr, nx, dy.ptr, ny), lib)
     return dy.numpy()
+
+
+def bfun3_route(shape, nvec=1, dtype=np.float64):
+    """How the product is formed (ttf_bfun3_route): 'chain', 'fused' or 'small'."""
+    lib = load()
+    route = C.c_int()
+    kind = {"d": b"d", "f": b"s", "D": b"z", "F": b"c"}[np.dtype(dtype).char]
+    check(lib.ttf_bfun3_route(kind, *shape, nvec, C.byref(route)), lib)
+    return ("chain", "fused", "small")[route.value]
 
 
 def phi_left(shape, phi1, A, x, y, complex_=False):
