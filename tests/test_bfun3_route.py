@@ -42,3 +42,27 @@ def test_refusals():
         assert lib.ttf_bfun3_route(kind, *sizes, nvec, ttfort.C.byref(out) if out is not None else None) != 0
         lib.ttf_clear_error()
     assert route.value == 7
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("left,n,right,ra,nvec", [(512, 2, 2, 3, 1), (512, 2, 1, 3, 1), (384, 2, 4, 5, 1), (400, 2, 8, 3, 1)])
+def test_few_large_groups_spread(dtype, left, n, right, ra, nvec):
+    """A long left rank and a short right one would leave the one-launch
+    kernel a work-group or a few, each with the whole of Phi1 to read: the
+    product spreads over the chip the other way."""
+    shape = (left, n, right, left, n, right, ra, ra)
+    assert ttfort.bfun3_route(shape, nvec, dtype) != "small"
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("left,n,right,ra,nvec", [(2, 2, 400, 5, 1), (4, 2, 400, 3, 1), (64, 2, 1, 5, 1), (64, 2, 64, 5, 1),
+                                                  (128, 2, 4, 5, 1), (32, 2, 32, 5, 8)])
+def test_many_or_small_groups_stay(dtype, left, n, right, ra, nvec):
+    shape = (left, n, right, left, n, right, ra, ra)
+    assert ttfort.bfun3_route(shape, nvec, dtype) == "small"
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+def test_more_groups_than_a_batch(dtype):
+    """The chains take at most 65535 products in a batch."""
+    assert ttfort.bfun3_route((1, 2, 1, 1, 2, 70000, 2, 2), 1, dtype) == "small"

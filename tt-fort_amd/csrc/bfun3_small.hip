@@ -15,7 +15,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 namespace ttf {
 
@@ -184,27 +186,85 @@ bool small_enabled() {
   return on;
 }
 
-// Where the one launch is the faster way: up to a number of multiply-adds
-// over all work-groups (columns as padded), past which the matrix cores'
-// tiles win.  Measured against the other path (us, other -> this), MPO rank
-// 5, n = 2, one vector unless said:
-//   f64   rank 2: 11.9 -> 4.7, 32: 13.7 -> 6.8, 64: 16.6 -> 8.6, 128: 29.1 ->
-//         18.8; 6 vectors at 64: 17.0 -> 12.7 (31e6), at 96: 26.0 -> 35.1
-//         (106e6); n = 4, rank 4, 6 vectors at 64: 16.2 -> 16.9 (63e6)
-//   f32   32: 15.5 -> 6.0, 128: 21.1 -> 13.7; 6 vectors at 96: 21.9 -> 20.1
-//         (106e6); n = 4, rank 4, 6 vectors at 96: 26.7 -> 27.0 (212e6)
-//   c128  32: 19.4 -> 7.6, 64: 21.8 -> 10.1, 128: 67.5 -> 24.5 (42e6); n = 4,
-//         rank 4 at 128: 61.0 -> 61.0 (84e6)
-//   c64   64: 17.9 -> 9.3, 128: 47.5 -> 22.5; n = 4, rank 4 at 128: 42.4 ->
-//         31.3 (84e6)
+// Where the one launch is the faster way: both ways' times estimated in us.
+//
+// A work-group streams its vector and all of phi1 through one CU, so its
+// time goes with the elements it loads, its multiply-adds (columns as padded)
+// and those of the middle stage, whose operands come one by one; with more
+// than 256 work-groups times the rounds.  A limit on the launch's total alone
+// let work-groups of any size through: (left rank, n, right rank, operator
+// rank) = (512, 2, 2, 3) in f64 took 92 us where the other way takes 18, (512,
+// 2, 1, 5) in f32 135 against 17.
+//
+// The other way in real types is the fused kernel or a chain of tuned
+// products: a few launches, and more with the total of multiply-adds.  In
+// complex types it is three products of fixed tiles (zgemm_plan), each the
+// chain of its K or rounds of it.
+//
+// The constants are least squares over 4300 shapes of the four types (ranks
+// 1 to 512, both sides equal or not, modes and operator ranks 1 to 8, 1 to 8
+// vectors; rms error 14 to 17 % for this kernel, 6 % for the complex chains)
+// and hold up to a total of multiply-adds, past which the matrix cores' tiles
+// are the rule.  Against the faster way of each shape below it the choice
+// loses 0.4 % on average in f64, 0.3 in f32, 0.1 in c128 and 0.4 in c64 (the
+// total alone: 22, 25, 3 and 11 %); at worst it takes 1.3 times the other
+// way's time in real types, 1.2 in c128 and 1.6 in c64.  Measured (us, other way
+// -> this), operator rank 5, n = 2, one vector unless said, ranks on both
+// sides or left x right:
+//   f64   2: 11.9 -> 4.6; 64: 16.5 -> 8.5; 128: 29.2 -> 18.6; 128 x 4: 22.8 ->
+//         15.0; 4 x 400, operator rank 3: 24.3 -> 11.4; other way: 256 x 4: 27.1
+//         against 42.8
+//   f32   64: 23.6 -> 7.0; 128: 27.8 -> 13.5; 128 x 4: 23.0 -> 10.3; other way:
+//         400 x 4, operator rank 3: 21.0 against 41.1
+//   c128  64: 21.9 -> 10.2; 128 x 4: 19.8 -> 15.7; other way: 256 x 1, operator
+//         rank 3: 19.6 against 27.1
+//   c64   64: 17.9 -> 9.3; 128 x 64: 23.7 -> 18.4; other way: 512 x 2, operator
+//         rank 3: 29.6 against 101
+struct SmallCost {
+  double start, load, mac, mid, round;
+};
+template <typename T> constexpr SmallCost kSmall = {5.3, 7.3e-5, 1.5e-5, 1.2e-4, 1.9};
+template <> constexpr SmallCost kSmall<float> = {5.2, 3.3e-5, 1.4e-5, 5.7e-5, 1.3};
+template <> constexpr SmallCost kSmall<hipDoubleComplex> = {5.7, 0.0, 5.7e-5, 1.6e-4, 2.4};
+template <> constexpr SmallCost kSmall<hipFloatComplex> = {5.6, 3.7e-5, 3.2e-5, 1.1e-4, 2.0};
+
+// A complex product: `k32` per k of a 32-wide tile's chain, `more32` of it for
+// each further round, `k64` per k and round of 64-wide tiles, `split` for a
+// second launch, `wgs` per 256 work-groups.
+struct ZCost {
+  double start, k32, more32, k64, split, wgs;
+};
+template <typename T> constexpr ZCost kZ = {3.0, 0.068, 0.068, 0.16, 3.2, 2.2};
+template <> constexpr ZCost kZ<hipFloatComplex> = {3.0, 0.046, 0.024, 0.10, 2.7, 1.1};
+
+template <typename T>
+double zgemm_us(int M, int N, int K, int nbatch) {
+  const ZCost c = kZ<T>;
+  const ZPlan p = zgemm_plan(M, N, K, nbatch);
+  const double per = std::ceil((double)K / p.ks), rounds = (double)p.tiles * nbatch * p.ks / 256;
+  const double sums = p.bm == 32 ? (c.k32 + c.more32 * std::max(0.0, rounds - 1)) * per : c.k64 * per * std::ceil(rounds);
+  return c.start + sums + (p.ks > 1 ? c.split : 0.0) + c.wgs * rounds;
+}
+
 template <typename T> constexpr double kMostMacs = 1.2e8;
 template <> constexpr double kMostMacs<double> = 5e7;
 template <> constexpr double kMostMacs<hipDoubleComplex> = 6e7;
 
 template <typename T>
-bool faster_small(const Shape& s, int nvec, int A2, int N) {
-  const double per = (double)s.rx1 * s.m * s.rx2 * A2 + (double)s.ry1 * s.rx1 * s.ra1 * N;
-  return per * s.ry2 * nvec <= kMostMacs<T>;
+bool faster_small(const Shape& s, int nvec, bool core, int A2, int N) {
+  const double groups = (double)s.ry2 * nvec, K3 = (double)s.rx1 * s.ra1;
+  const double wide1 = (double)s.rx1 * s.m * s.rx2, wide3 = s.ry1 * K3, macs = wide1 * A2 + wide3 * N;
+  if (macs * groups > kMostMacs<T>) return false;
+  if (groups > 65535) return true;   // the chains take no more products in one batch
+  const SmallCost c = kSmall<T>;
+  const double own = c.load * (wide1 + wide3) + c.mac * macs + (core ? c.mid * K3 * N * s.m * s.ra2 : 0.0);
+  const double rounds = std::max(1.0, groups / 256);
+  const double small = c.start + own * rounds + c.round * (rounds - 1);
+  if (std::is_same<T, double>::value) return small <= 17.5 + 1.5e-7 * macs * groups;
+  if (std::is_same<T, float>::value) return small <= 14.5 + 8e-8 * macs * groups;
+  double other = zgemm_us<T>(s.rx1 * s.m, s.ra2 * s.ry2, s.rx2, nvec);
+  if (core) other += zgemm_us<T>(s.rx1, s.ra1 * s.n, s.m * s.ra2, s.ry2 * nvec);
+  return small <= other + zgemm_us<T>(s.ry1, s.n * s.ry2, s.rx1 * s.ra1, nvec);
 }
 
 template <typename T, int A2, int N>
@@ -231,19 +291,19 @@ void launch(const SmallArgs<T>& a, int N, unsigned grid, size_t lds, hipStream_t
 }  // namespace
 
 template <typename T>
-bool bfun3_small_fits(const Shape& s, int nvec) {
+bool bfun3_small_fits(const Shape& s, int nvec, bool core) {
   if (!small_enabled() || nvec < 1 || s.ra2 > kMaxCols || s.n > kMaxCols) return false;
   const int64_t R1 = (int64_t)s.rx1 * s.m, K3 = (int64_t)s.rx1 * s.ra1;
   if (R1 > 2048 || K3 > 4096 || s.ry1 > 2048) return false;
   const int A2 = bucket(s.ra2), N = bucket(s.n);
-  return faster_small<T>(s, nvec, A2, N) && lds_need<T>(s, A2, N) <= kLdsBytes &&
-         (int64_t)s.ry2 * nvec <= 0x7fffffff / kNT;
+  return (int64_t)s.ry2 * nvec <= 0x7fffffff / kNT && lds_need<T>(s, A2, N) <= kLdsBytes &&
+         faster_small<T>(s, nvec, core, A2, N);
 }
 
 template <typename T>
 bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
                  int64_t ldy, hipStream_t st) {
-  if (!bfun3_small_fits<T>(s, nvec)) return false;
+  if (!bfun3_small_fits<T>(s, nvec, A != nullptr)) return false;
   const int A2 = bucket(s.ra2), N = bucket(s.n);
   const size_t lds = lds_need<T>(s, A2, N);
   SmallArgs<T> a{s.rx1, s.m, s.rx2, s.ry1, s.n, s.ry2, s.ra1, s.ra2, phi1, A, phi2, x, ldx, y, ldy};
@@ -258,10 +318,10 @@ bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* p
   return true;
 }
 
-template bool bfun3_small_fits<double>(const Shape&, int);
-template bool bfun3_small_fits<float>(const Shape&, int);
-template bool bfun3_small_fits<hipDoubleComplex>(const Shape&, int);
-template bool bfun3_small_fits<hipFloatComplex>(const Shape&, int);
+template bool bfun3_small_fits<double>(const Shape&, int, bool);
+template bool bfun3_small_fits<float>(const Shape&, int, bool);
+template bool bfun3_small_fits<hipDoubleComplex>(const Shape&, int, bool);
+template bool bfun3_small_fits<hipFloatComplex>(const Shape&, int, bool);
 template bool bfun3_small<double>(const Shape&, int, const double*, const double*, const double*, const double*,
                                   int64_t, double*, int64_t, hipStream_t);
 template bool bfun3_small<float>(const Shape&, int, const float*, const float*, const float*, const float*, int64_t,

@@ -32,8 +32,9 @@ bool bfun3_fused_fits(const Shape& s, int nvec);
 // the faster way, unless TTF_BFUN3_SMALL is 0; false leaves y untouched.
 // A == nullptr stands for the identity (m = n = 1, ra1 = ra2).  x and y must
 // not overlap.  T: double, float, hipDoubleComplex, hipFloatComplex.
+// bfun3_small_fits gives the choice alone (core: A is not nullptr).
 template <typename T>
-bool bfun3_small_fits(const Shape& s, int nvec);
+bool bfun3_small_fits(const Shape& s, int nvec, bool core = true);
 template <typename T>
 bool bfun3_small(const Shape& s, int nvec, const T* phi1, const T* A, const T* phi2, const T* x, int64_t ldx, T* y,
                  int64_t ldy, hipStream_t st);

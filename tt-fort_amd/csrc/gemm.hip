@@ -439,29 +439,31 @@ template size_t gemm_workspace<float>(const GemmOp<float>&);
 template void gemm_launch_ws<double>(GemmOp<double>, double*, size_t, hipStream_t);
 template void gemm_launch_ws<float>(GemmOp<float>, float*, size_t, hipStream_t);
 
+ZPlan zgemm_plan(int M, int N, int K, int nbatch) {
+  ZPlan p;
+  p.bm = ceil_div(M, 64) * ceil_div(N, 64) * (int64_t)nbatch >= 128 ? 64 : 32;
+  p.tiles = ceil_div(M, p.bm) * ceil_div(N, p.bm);
+  // few work-groups with a long K: slices of K in parallel (at least 48 deep
+  // each), summed by a second launch
+  p.ks = 1;
+  if (p.bm == 32 && p.tiles * nbatch < 32 && K >= 128)
+    p.ks = std::max(1, (int)std::min<int64_t>({8, K / 48, ceil_div(64, p.tiles * nbatch)}));
+  return p;
+}
+
 template <typename R>
 static void zgemm_launch_t(ZGemmOpT<R> op, hipStream_t st) {
   typedef typename CplxT<R>::type C_t;
   if (op.M <= 0 || op.N <= 0 || op.nbatch <= 0) return;
   if (op.nb0 <= 0) op.nb0 = 1;
   TTF_REQUIRE(op.nbatch <= 65535, "zgemm: batch count %d exceeds the grid limit", op.nbatch);
-  const int bm = ceil_div(op.M, 64) * ceil_div(op.N, 64) * (int64_t)op.nbatch >= 128 ? 64 : 32;
-  int64_t tiles = ceil_div(op.M, bm) * ceil_div(op.N, bm);
-  // few work-groups with a long K: slices of K in parallel (at least 48 deep
-  // each), summed by a second launch
-  op.ksplit = 1;
-  op.work = nullptr;
-  if (bm == 32 && tiles * op.nbatch < 32 && op.K >= 128) {
-    const int ks = (int)std::min<int64_t>({8, op.K / 48, ceil_div(64, tiles * op.nbatch)});
-    if (ks > 1) {
-      op.ksplit = ks;
-      op.work = (C_t*)arena(kArenaSplitK, sizeof(C_t) * (size_t)ks * op.nbatch * (size_t)op.M * op.N);
-    }
-  }
-  dim3 grid((unsigned)tiles, (unsigned)op.nbatch, (unsigned)op.ksplit);
+  const ZPlan p = zgemm_plan(op.M, op.N, op.K, op.nbatch);
+  op.ksplit = p.ks;
+  op.work = p.ks > 1 ? (C_t*)arena(kArenaSplitK, sizeof(C_t) * (size_t)p.ks * op.nbatch * (size_t)op.M * op.N) : nullptr;
+  dim3 grid((unsigned)p.tiles, (unsigned)op.nbatch, (unsigned)op.ksplit);
   // 32x32 tiles come with few work-groups, each one's K loop latency-bound
   // on its global loads: a 32-deep K chunk halves the trips
-  if (bm == 64)
+  if (p.bm == 64)
     hipLaunchKernelGGL((zgemm_mfma_kernel<R, 64, 64>), grid, dim3(256), 0, st, op);
   else if (op.K > 16)
     hipLaunchKernelGGL((zgemm_mfma_kernel<R, 32, 32, 32>), grid, dim3(256), 0, st, op);

@@ -697,6 +697,12 @@ size_t gemm_workspace(const GemmOp<T>& op);
 template <typename T>
 void gemm_launch_ws(GemmOp<T> op, T* ws, size_t ws_cap, hipStream_t st);
 void zgemm_launch(ZGemmOp op, hipStream_t st);
+// The tiles (bm x bm, `tiles` per batch) and the split of K of a complex product.
+struct ZPlan {
+  int bm, ks;
+  int64_t tiles;
+};
+ZPlan zgemm_plan(int M, int N, int K, int nbatch);
 void cgemm_launch(CGemmOp op, hipStream_t st);
 
 // While on, gemm_launch on this thread runs no tuning timings (for code
