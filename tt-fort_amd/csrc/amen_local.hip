@@ -48,7 +48,7 @@ __global__ void axpby_kernel(int64_t n, double a, const double* __restrict__ x, 
 // (tt_linalg.f90:397-491).  d1(b1, a1) = Phi1(b1, b1, a1), d2(b2, a2) =
 // Phi2(b2, a2, b2); A(a1, i, j, a2).
 //  'c': block (b1, b2) of size n: M(i, j) = sum d1(b1,a1) A(a1,i,j,a2) d2(b2,a2),
-//       stored at (b2 + rx2 b1) n^2 (layout (n, n, rx2, rx1)), formed as a product (jac_gen);
+//       stored at (b2 + rx2 b1) n^2 (layout (n, n, rx2, rx1)), formed as two products (jac_gen);
 //  'l': block b2 of size rx1 n: M((c1,i),(b1,j)) = sum Phi1(c1,b1,a1) A d2(b2,a2);
 //  'r': block b1 of size n rx2: M((i,c2),(j,b2)) = sum d1(b1,a1) A Phi2(b2,a2,c2).
 __global__ void jac_blocks_kernel(char type, int rx1, int n, int rx2, int ra1, int ra2,
@@ -86,28 +86,6 @@ __global__ void jac_blocks_kernel(char type, int rx1, int n, int rx2, int ra1, i
       }
     }
     M[e] = s;
-  }
-}
-
-// The two operands of the 'c' blocks as one product over the bond indices,
-//   M((i,j), b) = sum_{a1,a2} P((i,j), a1 + ra1 a2) D(a1 + ra1 a2, b),
-// b = b2 + rx2 b1: P is A with its bond indices last, D(., b) = d1(b1, a1)
-// d2(b2, a2).  One thread per entry of P, then of D.
-__global__ __launch_bounds__(256) void jac_c_operands_kernel(int rx1, int n, int rx2, int ra1, int ra2,
-                                                             const double* __restrict__ Phi1,
-                                                             const double* __restrict__ A,
-                                                             const double* __restrict__ Phi2,
-                                                             double* __restrict__ P, double* __restrict__ D) {
-  const int64_t nn = (int64_t)n * n, np = nn * ra1 * ra2, nk = (int64_t)ra1 * ra2;
-  const int64_t total = np + nk * rx1 * rx2;
-  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
-    if (e < np) {
-      const int64_t ij = e % nn, k = e / nn, a1 = k % ra1, a2 = k / ra1;
-      P[e] = A[a1 + ra1 * (ij + nn * a2)];
-    } else {
-      const int64_t f = e - np, k = f % nk, b = f / nk, a1 = k % ra1, a2 = k / ra1, b2 = b % rx2, b1 = b / rx2;
-      D[f] = Phi1[b1 + rx1 * (b1 + rx1 * a1)] * Phi2[b2 + rx2 * (a2 + ra2 * b2)];
-    }
   }
 }
 
@@ -363,23 +341,41 @@ void jac_gen(char type, int rx1, int n, int rx2, int ra1, int ra2, const double*
   TTF_REQUIRE(nblk <= 0x7fffffff, "djac_gen: too many blocks");
   const int64_t total = (int64_t)bs * bs * nblk;
   if (type == 'c') {
-    // every entry is a sum over the ra1 ra2 bond pairs, so the blocks are a
-    // product of n^2 x (ra1 ra2) by (ra1 ra2) x (rx1 rx2) on the matrix
-    // cores, bound by writing the blocks: 4096 blocks of order 64 with 36
-    // bond pairs take 46 us, where one thread per entry took 696.  Entries
-    // (i, j) and (j, i) are the same sums in the same order, so the blocks
-    // of a symmetric operator stay exactly symmetric.
-    const int64_t nk = (int64_t)ra1 * ra2, nn = (int64_t)n * n;
-    double* P = (double*)arena(kArenaSolver2, sizeof(double) * (size_t)(nk * (nn + nblk)));
-    double* D = P + nk * nn;
-    hipLaunchKernelGGL(jac_c_operands_kernel, dim3(grid_for(nk * (nn + nblk))), dim3(256), 0, st, rx1, n, rx2, ra1,
-                       ra2, Phi1, A, Phi2, P, D);
-    TTF_HIP(hipGetLastError());
-    // the ranks change from one local problem to the next: no tuning runs
-    // for products that may be formed once
-    GemmOp<double> g = colmajor<double>('N', 'N', (int)nn, (int)nblk, (int)nk, 1.0, P, nn, D, nk, 0.0, jacs, nn);
-    const size_t ws = gemm_workspace(g);
-    gemm_launch_ws(g, ws ? (double*)arena(kArenaSplitK, sizeof(double) * ws) : nullptr, ws, st);
+    // as two products on the matrix cores, in the order of the sums above,
+    //   T((i,j), a2, b1) = sum_a1 A(a1, (i,j), a2) d1(b1, a1)
+    //   M((i,j), b2, b1) = sum_a2 T((i,j), a2, b1) d2(b2, a2),
+    // with the diagonals of Phi1 and Phi2 read in place (strides rx1 + 1 and
+    // 1 + rx2 ra2), bound by writing the blocks.  4096 blocks of order 64 with
+    // operator ranks 6, inverses included: 1214 us with one thread per entry,
+    // 216 so; one product over the bond pairs took 226, and its second operand
+    // ra1 ra2 times the blocks in scratch.  Entries (i, j) and (j, i) are the same sums in the same order, so the
+    // blocks of a symmetric operator stay exactly symmetric.  T is made for
+    // as many b1 at a time as 64 MB hold.  The ranks change from one local
+    // problem to the next: no tuning runs for products that may be formed
+    // once.
+    const int64_t nn = (int64_t)n * n, per = nn * ra2;
+    const int64_t most = std::min<int64_t>({rx1, 65535, std::max<int64_t>(1, ((int64_t)1 << 23) / per)});
+    double* T = (double*)arena(kArenaSolver2, sizeof(double) * (size_t)(per * most));
+    auto product = [&](const GemmOp<double>& g) {
+      const size_t ws = gemm_workspace(g);
+      gemm_launch_ws(g, ws ? (double*)arena(kArenaSplitK, sizeof(double) * ws) : nullptr, ws, st);
+    };
+    for (int64_t b1 = 0; b1 < rx1; b1 += most) {
+      const int nb = (int)std::min<int64_t>(most, rx1 - b1);
+      GemmOp<double> g{};
+      g.M = (int)nn; g.N = nb; g.K = ra1;
+      g.A = A; g.sAi = ra1; g.sAk = 1; g.sAb0 = (int64_t)ra1 * nn;
+      g.B = Phi1 + b1 * (rx1 + 1); g.sBk = (int64_t)rx1 * rx1; g.sBj = rx1 + 1;
+      g.C = T; g.sCi = 1; g.sCj = per; g.sCb0 = nn;
+      g.nb0 = ra2; g.nbatch = ra2; g.alpha = 1.0; g.beta = 0.0; g.ksplit = 1;
+      product(g);
+      g.M = (int)nn; g.N = rx2; g.K = ra2;
+      g.A = T; g.sAi = 1; g.sAk = nn; g.sAb0 = per;
+      g.B = Phi2; g.sBk = rx2; g.sBj = 1 + (int64_t)rx2 * ra2;
+      g.C = jacs + nn * rx2 * b1; g.sCi = 1; g.sCj = nn; g.sCb0 = nn * rx2;
+      g.nb0 = nb; g.nbatch = nb;
+      product(g);
+    }
   } else {
     hipLaunchKernelGGL(jac_blocks_kernel, dim3(grid_for(total)), dim3(256), 0, st, type, rx1, n, rx2, ra1, ra2,
                        Phi1, A, Phi2, jacs);
