@@ -348,11 +348,11 @@ void jac_gen(char type, int rx1, int n, int rx2, int ra1, int ra2, const double*
     // 1 + rx2 ra2), bound by writing the blocks.  4096 blocks of order 64 with
     // operator ranks 6, inverses included: 1214 us with one thread per entry,
     // 216 so; one product over the bond pairs took 226, and its second operand
-    // ra1 ra2 times the blocks in scratch.  Entries (i, j) and (j, i) are the same sums in the same order, so the
-    // blocks of a symmetric operator stay exactly symmetric.  T is made for
-    // as many b1 at a time as 64 MB hold.  The ranks change from one local
-    // problem to the next: no tuning runs for products that may be formed
-    // once.
+    // ra1 ra2 times the blocks in scratch.  Entries (i, j) and (j, i) are the
+    // same sums in the same order, so the blocks of a symmetric operator stay
+    // exactly symmetric.  T is made for as many b1 at a time as 64 MB hold.
+    // The ranks change from one local problem to the next: no tuning runs for
+    // products that may be formed once.
     const int64_t nn = (int64_t)n * n, per = nn * ra2;
     const int64_t most = std::min<int64_t>({rx1, 65535, std::max<int64_t>(1, ((int64_t)1 << 23) / per)});
     double* T = (double*)arena(kArenaSolver2, sizeof(double) * (size_t)(per * most));
