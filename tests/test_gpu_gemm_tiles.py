@@ -62,3 +62,15 @@ def test_gemm_tile_edges(ttlib, side, dims):
     assert np.all(np.abs(aligned - ref) <= bound)
     shifted, _, _ = _run(side, dims, 1)
     assert np.array_equal(aligned, shifted)   # the same sums in the same order
+
+
+def test_tuning_follows_the_load_mode(ttlib):
+    """A tile timed on aligned operands is not taken over for operands that
+    are read element by element, nor the other way round; each is tuned once."""
+    dims = (200, 72, 136, 3, 104)   # sizes no other test uses
+    tuned = []
+    for shift in (0, 1, 0, 1):
+        before = ttlib.ttf_autotune_count()
+        _run("left", dims, shift)
+        tuned.append(ttlib.ttf_autotune_count() - before)
+    assert tuned[0] > 0 and tuned[1] > 0 and tuned[2:] == [0, 0]

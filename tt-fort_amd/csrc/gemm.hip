@@ -110,6 +110,33 @@ struct Tile {
 static const Tile kTiles[] = {{128, 64, 256, 92}, {64, 96, 512, 90}, {64, 80, 256, 84}, {64, 64, 256, 86},
                               {64, 32, 256, 82},  {32, 32, 256, 70}, {32, 16, 64, 45}};
 
+// Whether an operand's offsets inside a tile (at most 128 rows and 64 of k)
+// fit 32 bits.
+template <typename T>
+static bool operand_near(int64_t s_row, int64_t s_k) {
+  const int64_t most = ((int64_t)1 << 32) / (int64_t)sizeof(T);
+  return s_row >= 0 && s_k >= 0 && s_row < most && s_k < most && 128 * s_row + 64 * s_k < most;
+}
+
+// Whether an operand (rows x K, strides s_row, s_k, batch strides) can be
+// read 16 bytes at a time along its contiguous direction: pointer, other
+// strides and the extent of that direction all whole multiples of 16 bytes.
+template <typename T>
+static bool operand_aligned(const T* p, int64_t s_row, int64_t s_k, int64_t sb0, int64_t sb1, int rows, int K) {
+  constexpr int V = 16 / (int)sizeof(T);
+  if ((reinterpret_cast<uintptr_t>(p) & 15) != 0 || sb0 % V != 0 || sb1 % V != 0) return false;
+  if (s_row == 1) return s_k % V == 0 && rows % V == 0;
+  return s_k == 1 && s_row % V == 0 && K % V == 0;
+}
+
+template <typename T>
+static LoadMode load_mode(const GemmOp<T>& op) {
+  if (!operand_near<T>(op.sAi, op.sAk) || !operand_near<T>(op.sBj, op.sBk)) return kWide;
+  const bool va = operand_aligned(op.A, op.sAi, op.sAk, op.sAb0, op.sAb1, op.M, op.K);
+  const bool vb = operand_aligned(op.B, op.sBj, op.sBk, op.sBb0, op.sBb1, op.N, op.K);
+  return va && vb ? kVecBoth : (va ? kVecA : (vb ? kVecB : kScalar));
+}
+
 struct Key {
   int type, M, N, K, nbatch, flags;
   bool operator==(const Key& o) const {
@@ -124,6 +151,21 @@ struct KeyHash {
     return h;
   }
 };
+
+template <typename T> static int type_id();
+template <> int type_id<double>() { return 0; }
+template <> int type_id<float>() { return 1; }
+
+// A product's key: sizes, which directions are contiguous, and how its tiles
+// read their operands, since one tile's time differs between the modes (both
+// operands in 16-byte loads is 0, the mode of tables without one).
+template <typename T>
+static Key key_of(const GemmOp<T>& op) {
+  const LoadMode m = load_mode(op);
+  const int mode = m == kVecBoth ? 0 : (m == kVecA ? 1 : (m == kVecB ? 2 : (m == kScalar ? 3 : 4)));
+  return {type_id<T>(), op.M, op.N, op.K, op.nbatch,
+          (op.sAi == 1 ? 1 : 0) | (op.sBj == 1 ? 2 : 0) | (op.sCi == 1 ? 4 : 0) | (mode << 3)};
+}
 
 namespace {
 std::mutex g_tune_mu;
@@ -256,41 +298,23 @@ static void launch_tiles(const GemmOp<T>& op, const Cfg& c, hipStream_t st) {
   }
 }
 
-// Whether an operand's offsets inside a tile (at most 128 rows and 64 of k)
-// fit 32 bits.
-template <typename T>
-static bool operand_near(int64_t s_row, int64_t s_k) {
-  const int64_t most = ((int64_t)1 << 32) / (int64_t)sizeof(T);
-  return s_row >= 0 && s_k >= 0 && s_row < most && s_k < most && 128 * s_row + 64 * s_k < most;
-}
-
-// Whether an operand (rows x K, strides s_row, s_k, batch strides) can be
-// read 16 bytes at a time along its contiguous direction: pointer, other
-// strides and the extent of that direction all whole multiples of 16 bytes.
-template <typename T>
-static bool operand_aligned(const T* p, int64_t s_row, int64_t s_k, int64_t sb0, int64_t sb1, int rows, int K) {
-  constexpr int V = 16 / (int)sizeof(T);
-  if ((reinterpret_cast<uintptr_t>(p) & 15) != 0 || sb0 % V != 0 || sb1 % V != 0) return false;
-  if (s_row == 1) return s_k % V == 0 && rows % V == 0;
-  return s_k == 1 && s_row % V == 0 && K % V == 0;
-}
-
 template <typename T>
 static void launch_cfg(GemmOp<T> op, const Cfg& c, hipStream_t st) {
   op.ksplit = c.ks;
   // column-contiguous outputs (and the column-major split-K slices) take the
   // swapped-fragment variant, whose lanes store consecutive rows; the other
   // outputs are few, and small, and read element by element
-  const bool ct = op.ksplit > 1 || op.sCi == 1;
-  const bool near = operand_near<T>(op.sAi, op.sAk) && operand_near<T>(op.sBj, op.sBk);
-  const bool va = operand_aligned(op.A, op.sAi, op.sAk, op.sAb0, op.sAb1, op.M, op.K);
-  const bool vb = operand_aligned(op.B, op.sBj, op.sBk, op.sBb0, op.sBb1, op.N, op.K);
-  if (!ct) launch_tiles<T, false, kWide>(op, c, st);
-  else if (!near) launch_tiles<T, true, kWide>(op, c, st);
-  else if (va && vb) launch_tiles<T, true, kVecBoth>(op, c, st);
-  else if (va) launch_tiles<T, true, kVecA>(op, c, st);
-  else if (vb) launch_tiles<T, true, kVecB>(op, c, st);
-  else launch_tiles<T, true, kScalar>(op, c, st);
+  if (op.ksplit == 1 && op.sCi != 1) {
+    launch_tiles<T, false, kWide>(op, c, st);
+  } else {
+    switch (load_mode(op)) {
+      case kWide: launch_tiles<T, true, kWide>(op, c, st); break;
+      case kVecBoth: launch_tiles<T, true, kVecBoth>(op, c, st); break;
+      case kVecA: launch_tiles<T, true, kVecA>(op, c, st); break;
+      case kVecB: launch_tiles<T, true, kVecB>(op, c, st); break;
+      default: launch_tiles<T, true, kScalar>(op, c, st); break;
+    }
+  }
   TTF_HIP(hipGetLastError());
   if (op.ksplit > 1) {
     int64_t total = (int64_t)op.M * op.N * op.nbatch;
@@ -347,10 +371,6 @@ static Cfg tune(const GemmOp<T>& op0, hipStream_t st) {
   return best;
 }
 
-template <typename T> static int type_id();
-template <> int type_id<double>() { return 0; }
-template <> int type_id<float>() { return 1; }
-
 template <typename T>
 void gemm_launch(GemmOp<T> op, hipStream_t st) {
   if (op.M <= 0 || op.N <= 0 || op.nbatch <= 0) return;
@@ -375,8 +395,7 @@ void gemm_launch(GemmOp<T> op, hipStream_t st) {
     return;
   }
   const double flops = 2.0 * op.M * op.N * (double)op.K * op.nbatch;
-  Key key{type_id<T>(), op.M, op.N, op.K, op.nbatch,
-          (op.sAi == 1 ? 1 : 0) | (op.sBj == 1 ? 2 : 0) | (op.sCi == 1 ? 4 : 0)};
+  const Key key = key_of(op);
   Cfg c;
   bool have = false;
   {
@@ -415,8 +434,7 @@ void gemm_launch_ws(GemmOp<T> op, T* ws, size_t ws_cap, hipStream_t st) {
     gemm_launch(op, st);   // the panel kernel needs no workspace and is never tuned
     return;
   }
-  Key key{type_id<T>(), op.M, op.N, op.K, op.nbatch,
-          (op.sAi == 1 ? 1 : 0) | (op.sBj == 1 ? 2 : 0) | (op.sCi == 1 ? 4 : 0)};
+  const Key key = key_of(op);
   Cfg c = heuristic(op.M, op.N, op.K, op.nbatch);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
