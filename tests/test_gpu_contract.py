@@ -246,17 +246,30 @@ print(json.dumps({"rel": worst}))
     assert [ln for ln in lines if ln.startswith("0 256 640 128 ")] == pinned, lines
 
 
-@pytest.mark.parametrize("nvec", [1, 8, 16])
-def test_dbfun3_fused_matches_gemm_chain(ttlib, tmp_path, nvec):
-    """At the (128, 2, 128, R = 5) local shape the library runs the fused
-    one-launch kernel; the GEMM chain (TTF_BFUN3_FUSED=0, in a child
-    process) gives the same products to 1e-13 of the problem scale, and two
-    fused calls give identical bits (the two halves of the b1 range meet by
-    commutative additions onto zero)."""
-    import json
+def _child(tmp_path, code, *args, **env):
+    """Runs `code` in a process of its own (the kernels' switches are read
+    once) and returns the words of its last line."""
     import os
     import subprocess
     import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    head = ("import os, sys\nroot, d = sys.argv[1:3]\nsys.path[:0] = [root, os.path.join(root, 'tt-fort_amd')]\n"
+            "import numpy as np, ttfort\n")
+    r = subprocess.run([sys.executable, "-c", head + code, root, str(tmp_path)] + [str(a) for a in args],
+                       env=dict(os.environ, **env), capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout[-1000:] + r.stderr[-3000:]
+    return r.stdout.strip().splitlines()[-1].split()
+
+
+@pytest.mark.parametrize("nvec", [1, 8, 16])
+def test_dbfun3_fused_matches_gemm_chain(ttlib, tmp_path, nvec):
+    """At the (128, 2, 128, R = 5) local shape the library runs a one-launch
+    kernel: the vector kernel for one vector, the fused one for more.  The
+    fused kernel and the GEMM chain, each in a child process with the others
+    switched off, give the same products to 1e-13 of the problem scale, as
+    the library's own choice does, and two calls give identical bits (in the
+    fused kernel the two halves of the b1 range meet by commutative additions
+    onto zero)."""
     import ttfort
     shape = (128, 2, 128, 128, 2, 128, 5, 5)
     rng = np.random.default_rng(30 + nvec)
@@ -273,23 +286,46 @@ def test_dbfun3_fused_matches_gemm_chain(ttlib, tmp_path, nvec):
                                               d["x"].ptr, nx, dy.ptr, ny, 3, ttfort.C.byref(ms),
                                               ttfort.C.byref(fused)), lib)
     assert fused.value == 1
+    assert ttfort.bfun3_route(shape, nvec) == ("small" if nvec == 1 else "fused")
     y1 = dy.numpy().copy()
     y2 = ttfort.bfun3(shape, t["phi1"], t["A"], t["phi2"], t["x"], nvec=nvec)
     assert np.array_equal(y1, y2)
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     code = r'''
-import os, sys
-root, d, nvec = sys.argv[1], sys.argv[2], int(sys.argv[3])
-sys.path[:0] = [root, os.path.join(root, "tt-fort_amd")]
-import numpy as np
-import ttfort
+nvec, out = int(sys.argv[3]), sys.argv[4]
+shape = (128, 2, 128, 128, 2, 128, 5, 5)
 t = {k: np.load(os.path.join(d, k + ".npy")) for k in ("phi1", "A", "phi2", "x")}
-y = ttfort.bfun3((128, 2, 128, 128, 2, 128, 5, 5), t["phi1"], t["A"], t["phi2"], t["x"], nvec=nvec)
-np.save(os.path.join(d, "y_chain.npy"), y)
+y = [ttfort.bfun3(shape, t["phi1"], t["A"], t["phi2"], t["x"], nvec=nvec) for _ in range(2)]
+np.save(os.path.join(d, out), y[0])
+print(ttfort.bfun3_route(shape, nvec), np.array_equal(y[0], y[1]))
 '''
-    env = dict(os.environ, TTF_BFUN3_FUSED="0")
-    r = subprocess.run([sys.executable, "-c", code, root, str(tmp_path), str(nvec)], env=env,
-                       capture_output=True, text=True, timeout=600)
-    assert r.returncode == 0, r.stderr[-3000:]
+    env = dict(TTF_BFUN3_SMALL="0")
+    assert _child(tmp_path, code, nvec, "y_fused.npy", **env) == ["fused", "True"]
+    assert _child(tmp_path, code, nvec, "y_chain.npy", TTF_BFUN3_FUSED="0", **env)[0] == "chain"
     yc = np.load(tmp_path / "y_chain.npy")
     assert np.abs(y1 - yc).max() <= 1e-13 * _scale(shape, t)
+    assert np.abs(np.load(tmp_path / "y_fused.npy") - yc).max() <= 1e-13 * _scale(shape, t)
+
+
+def test_other_routes_match_oracle(ttlib, tmp_path):
+    """The shapes of this file that the one-launch vector kernel takes, with
+    that kernel switched off: the fused kernel's edges, and the GEMM chains of
+    the other types (FP32, complex64, complex128) against the oracle."""
+    code = r'''
+from tests import test_gpu_contract as c
+ttfort.check(ttfort.load().ttf_init(0))
+for shape in c.SHAPES:
+    for nvec in (1, 5, 8):
+        print(shape, nvec, flush=True)
+        assert ttfort.bfun3_route(shape, nvec) == "fused"
+        c.test_dbfun3(None, shape, nvec)
+    for dtype in (np.float32, np.complex64, np.complex128):
+        assert ttfort.bfun3_route(shape, 2, dtype) == "chain"
+for shape in c.SHAPES[2:]:
+    c.test_sbfun3_fp32(None, shape)
+    c.test_cbfun3_complex64(None, shape)
+for shape in c.SHAPES[:6]:
+    c.test_zbfun3_and_transp(None, shape)
+print("done")
+'''
+    assert _child(tmp_path, code, TTF_BFUN3_SMALL="0") == ["done"]
+

@@ -66,9 +66,9 @@ def test_gesvd_graded_relative_accuracy(ttlib):
 
 @pytest.mark.parametrize("n", [1, 2, 5, 24, 31, 32, 33, 48, 64])
 def test_syev_small(ttlib, n):
-    """Orders up to 32 take the slot-ordered Jacobi (one 2x2 block per
-    thread), 33 and above the double-buffered circle one; odd orders are
-    padded with a zero row."""
+    """Orders up to 60 take the slot-ordered Jacobi with its rotations a round
+    ahead (512 threads up to 32, 1024 past it), 61 to 64 the one in place; odd
+    orders are padded with a zero row."""
     import ttfort
     rng = np.random.default_rng(n)
     As = []
