@@ -342,17 +342,20 @@ __device__ double (*jacobi_sym_slots(double (*A)[LD], double (*B)[LD], double (*
   return A;
 }
 
-// The slot-ordered form for a block whose every wave owns 2x2 blocks (orders
-// 33 to 64 on 1024 threads): two barriers a round, updates in place.
-// Thread (kp, kq) owns the 2x2 block of slot pairs kp x kq; a round: each
-// thread loads its block and its two rows of the vectors' slot pair kq; the
-// diagonal-block threads compute the round's rotations and publish them;
-// after a barrier every thread applies its two rotations and stores the block
-// at the slots its contents move to.  Rotations taken a round ahead would run
-// beside the blocks of the same waves: up to 818 us against 534 us for a
-// solve of 1024 threads.  Working copies: the matrix in slot order in B, the
-// vectors (V with columns in slot order) in A; at the end V receives the
-// vectors in index order and A's diagonal the eigenvalues, and A is returned.
+// The slot-ordered form for a block that has no wave left for the rotations
+// (orders 61 to 64 on 1024 threads, 27 to 32 on 256): two barriers a round,
+// updates in place.  Thread (kp, kq) owns the 2x2 block of slot pairs kp x kq; a
+// round: each thread loads its block and its two rows of the vectors' slot
+// pair kq; the diagonal-block threads compute the round's rotations and
+// publish them; after a barrier every thread applies its two rotations and
+// stores the block at the slots its contents move to.  Rotations taken a round
+// ahead by waves that own blocks as well took 818 us against 534 for a solve
+// of order 64.  Where a wave is free the form above is the faster one or equal:
+// on 1024 threads order 60 takes 654 us in place and 547 with it, 48 303 and
+// 274, 44 251 and 254, 33 164 and 144.  Working copies: the matrix in slot
+// order in B, the vectors (V with columns in slot order) in A; at the end V
+// receives the vectors in index order and A's diagonal the eigenvalues, and A
+// is returned.
 template <int LD, class Go>
 __device__ double (*jacobi_sym_slots_inplace(double (*A)[LD], double (*B)[LD], double (*V)[LD], int n, int max_sweeps,
                                      const Go& go, int* flags, double small))[LD] {

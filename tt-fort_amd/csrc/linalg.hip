@@ -151,8 +151,8 @@ __device__ void write_sorted(double (*A)[LD], double (*V)[LD], int n, int desc, 
 
 // A thread per 2x2 block of the Jacobi rounds, and up to order 32 as many
 // again for the rotations and the vectors: 512 threads up to there, 1024 past
-// it (orders 33 to 64, up to 1068 us with 256 threads and four blocks each, up
-// to 534 us with 1024).
+// it (256 threads with four blocks each -> 1024: order 33 281 -> 145 us, 60 996
+// -> 485, 64 1069 -> 546).
 __global__ __launch_bounds__(1024) void syev_small_kernel(int n, double* Aall, double* wall,
                                                          double* Qall, int desc) {
   __shared__ double A[64][65], B[64][65];
@@ -620,9 +620,9 @@ __device__ inline void lds_gram8(const double* P, int rows, int ld, int n, doubl
 // rotations' relative tolerance, the skip and the convergence, as the
 // column form's dot products do.  `scale` (a power of two near 1 / ||W||_F^2)
 // keeps the squares of the Gram's entries in range, with small2 scaled alike.
-// 256 rows, 32 columns: 40.2 us with the column form -> 27.8 us; the number
-// of sweeps is unchanged.  Bound by the chain of the 31 rounds (37800 of
-// 62000 clocks; the Gram 9000, the update 7900, the loads 6000).
+// 256 rows, 32 columns: 40.2 us with the column form -> 27.3 us; the number
+// of sweeps is unchanged.  Bound by the chain of the 31 rounds (about 37000 of
+// 61000 clocks; the Gram 9000, the update 7900, the loads 6000).
 constexpr int kPairLd = 34;   // row stride of the 32 x 32 work matrices (jacobi.h: even)
 
 __global__ __launch_bounds__(512) void svd_pair_gram_kernel(int mw, int nw, int bsz, int nb, int round,
@@ -975,6 +975,9 @@ __global__ __launch_bounds__(64 * kQrWaves) void qr_panel_reg_kernel(int rows, i
   }
 }
 
+// Up to 1024 rows fit sixteen waves' registers.  The whole of ttf_dqr, LDS
+// panels -> register panels (us): 256 x 64 310 -> 157, 640 x 64 479 -> 209, 900
+// x 64 604 -> 230, 1024 x 32 330 -> 114, 1024 x 256 2230 -> 872.
 constexpr int kQrRegRows = 1024;
 // Columns per Householder panel of a p-row matrix: what the register panel
 // holds, or what fits the LDS budget of longer ones.
