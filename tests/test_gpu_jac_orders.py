@@ -1,8 +1,9 @@
 """Block-Jacobi 'c' blocks at the orders where the register tiles of the
 symmetric inverse change (16 TS = 32, 64, 128) and one past them, for
 operators whose blocks are positive definite, and for non-symmetric ones
-that take the pivoting inverse, with one and with many bond pairs, and more
-left indices than one slice of the blocks' intermediate holds.
+that take the pivoting inverse, with one and with many bond pairs, more left
+indices than one slice of the blocks' intermediate holds, and an operator
+rank past one batch of products.
 
 Against the oracle (LU-based): condition numbers are below 20, so 1e-10
 relative covers the rounding of both inverses at order 128.
@@ -18,7 +19,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("symmetric", [True, False])
 @pytest.mark.parametrize("rx1,n,rx2,ra1,ra2", [(1, 1, 1, 1, 1), (3, 2, 5, 1, 2), (5, 31, 4, 3, 3), (2, 32, 3, 2, 2),
                                                (3, 33, 2, 6, 6), (4, 64, 5, 6, 6), (2, 65, 2, 2, 3), (1, 127, 3, 2, 1),
-                                               (2, 128, 1, 2, 2), (40, 3, 33, 2, 2), (130, 64, 1, 1, 20)])
+                                               (2, 128, 1, 2, 2), (40, 3, 33, 2, 2), (130, 64, 1, 1, 20), (2, 1, 3, 1, 70000)])
 def test_djac_c_orders(ttlib, rx1, n, rx2, ra1, ra2, symmetric):
     import ttfort
     rng = np.random.default_rng(n)

@@ -364,11 +364,16 @@ void jac_gen(char type, int rx1, int n, int rx2, int ra1, int ra2, const double*
       const int nb = (int)std::min<int64_t>(most, rx1 - b1);
       GemmOp<double> g{};
       g.M = (int)nn; g.N = nb; g.K = ra1;
-      g.A = A; g.sAi = ra1; g.sAk = 1; g.sAb0 = (int64_t)ra1 * nn;
+      g.sAi = ra1; g.sAk = 1; g.sAb0 = (int64_t)ra1 * nn;
       g.B = Phi1 + b1 * (rx1 + 1); g.sBk = (int64_t)rx1 * rx1; g.sBj = rx1 + 1;
-      g.C = T; g.sCi = 1; g.sCj = per; g.sCb0 = nn;
-      g.nb0 = ra2; g.nbatch = ra2; g.alpha = 1.0; g.beta = 0.0; g.ksplit = 1;
-      product(g);
+      g.sCi = 1; g.sCj = per; g.sCb0 = nn;
+      g.alpha = 1.0; g.beta = 0.0; g.ksplit = 1;
+      for (int64_t a2 = 0; a2 < ra2; a2 += 65535) {   // a batch's limit
+        g.A = A + (int64_t)ra1 * nn * a2;
+        g.C = T + nn * a2;
+        g.nb0 = g.nbatch = (int)std::min<int64_t>(65535, ra2 - a2);
+        product(g);
+      }
       g.M = (int)nn; g.N = rx2; g.K = ra2;
       g.A = T; g.sAi = 1; g.sAk = nn; g.sAb0 = per;
       g.B = Phi2; g.sBk = rx2; g.sBj = 1 + (int64_t)rx2 * ra2;
